@@ -75,7 +75,9 @@ int su2_ctx_memory(su2_ctx* ctx, long long* live, long long* peak, long long* ca
 /* Tuning of the one-sided Jacobi SVD behind su2_svd_truncate and the DMRG
  * solves: column block width 16 or 32 (default 32), inner Jacobi sweeps per
  * visit of a pair 1..3 (default 1).  No counterpart in the reference; the
- * results agree to the SVD's own accuracy either way. */
+ * results agree to the SVD's own accuracy either way.  Blocks that fit one
+ * compute unit's LDS (up to 96 x 96) are decomposed there, whatever is set
+ * here or below. */
 int su2_ctx_set_svd_tuning(su2_ctx* ctx, int block_cols, int inner_sweeps);
 /* QR preconditioning of the Jacobi SVD: for every sector block with
  * min_k <= min(m, n) <= 2048 (min_k 2..2048, default 256; 0 turns it off),

@@ -12,6 +12,7 @@
 #include "common.hpp"
 #include "context.hpp"
 #include "precond.hpp"
+#include "small_svd.hpp"
 
 namespace su2 {
 
@@ -25,6 +26,7 @@ constexpr int MIN_SLICE_ROWS = 64;
 // of the block: they carry no direction, no pair with one of them holds the
 // iteration open, and the sweeps leave them out of the schedule.
 constexpr double kNoiseRel = 1e-13;
+constexpr double kTolAbs = 1e-14;   // rounding floor of a pair, relative to ||A||_F
 
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 
@@ -727,9 +729,9 @@ struct DevMem {
 
 }  // namespace
 
-int jacobi_svd_batched(Context& c, std::vector<JacobiBlock>& blocks, double tol, int max_sweeps,
-                       int block_cols, int inner_sweeps, double* worst_out,
-                       int precondition_min_k) {
+static int jacobi_svd_large(Context& c, const std::vector<JacobiBlock*>& blocks, double tol,
+                            int max_sweeps, int block_cols, int inner_sweeps, double* worst_out,
+                            int precondition_min_k) {
   if (worst_out) *worst_out = 0.0;
   hipStream_t st = c.stream();
   const int nb = (int)blocks.size();
@@ -745,9 +747,9 @@ int jacobi_svd_batched(Context& c, std::vector<JacobiBlock>& blocks, double tol,
   std::vector<int> L(nb), K(nb);
   std::vector<long long> noff(nb + 1, 0);
   for (int b = 0; b < nb; ++b) {
-    SU2_CHECK(blocks[b].m >= 1 && blocks[b].n >= 1, kErrArgument, "jacobi: empty block");
-    L[b] = std::max(blocks[b].m, blocks[b].n);
-    K[b] = std::min(blocks[b].m, blocks[b].n);
+    SU2_CHECK(blocks[b]->m >= 1 && blocks[b]->n >= 1, kErrArgument, "jacobi: empty block");
+    L[b] = std::max(blocks[b]->m, blocks[b]->n);
+    K[b] = std::min(blocks[b]->m, blocks[b]->n);
     noff[b + 1] = noff[b] + K[b];
   }
   const long long ncol = noff[nb];
@@ -757,7 +759,7 @@ int jacobi_svd_batched(Context& c, std::vector<JacobiBlock>& blocks, double tol,
   std::vector<std::unique_ptr<DevMem>> W2(nb), V2(nb);
   std::vector<double*> Wc(nb), Vc(nb), Wo(nb), Vo(nb);
   for (int b = 0; b < nb; ++b) {
-    JacobiBlock& J = blocks[b];
+    JacobiBlock& J = *blocks[b];
     W2[b].reset(new DevMem(c, sizeof(double) * (size_t)L[b] * K[b]));
     V2[b].reset(new DevMem(c, sizeof(double) * (size_t)K[b] * K[b]));
     Wc[b] = J.W;
@@ -937,11 +939,11 @@ int jacobi_svd_batched(Context& c, std::vector<JacobiBlock>& blocks, double tol,
       round_off[r] = (int)all.size();
       const int nj = (int)rounds[r].size();
       std::map<int, int> per_group;
-      for (const PairJob& j : rounds[r]) per_group[blocks[j.blk].group]++;
+      for (const PairJob& j : rounds[r]) per_group[blocks[j.blk]->group]++;
       int used = 1;
       for (PairJob& j : rounds[r]) {
         const int pmax =
-            std::min(MAX_SLICES, std::max(1, slice_target / per_group[blocks[j.blk].group]));
+            std::min(MAX_SLICES, std::max(1, slice_target / per_group[blocks[j.blk]->group]));
         j.P = std::max(1, std::min(pmax, L[j.blk] / MIN_SLICE_ROWS));
         used = std::max(used, j.P);
       }
@@ -987,13 +989,15 @@ int jacobi_svd_batched(Context& c, std::vector<JacobiBlock>& blocks, double tol,
         hipLaunchKernelGGL((gram_partial_kernel<16, 64, RCH>), dim3(nj * pm), dim3(64), 0, st,
                            (const BlockDesc*)ddesc.p, jr, pm, (double*)dgpart.p);
         hipLaunchKernelGGL((jacobi_rotate_kernel<16, 64>), dim3(nj * pm), dim3(64), 0, st,
-                           (const BlockDesc*)ddesc.p, jr, pm, (const double*)dgpart.p, tol, 1e-14,
+                           (const BlockDesc*)ddesc.p, jr, pm, (const double*)dgpart.p, tol,
+                           kTolAbs,
                            (unsigned long long*)doff.p, inner_sweeps);
       } else {
         hipLaunchKernelGGL((gram_partial_kernel<32, 1024, 64>), dim3(nj * pm), dim3(1024), 0, st,
                            (const BlockDesc*)ddesc.p, jr, pm, (double*)dgpart.p);
         hipLaunchKernelGGL((jacobi_rotate_kernel<32, 512>), dim3(nj * pm), dim3(512), 0, st,
-                           (const BlockDesc*)ddesc.p, jr, pm, (const double*)dgpart.p, tol, 1e-14,
+                           (const BlockDesc*)ddesc.p, jr, pm, (const double*)dgpart.p, tol,
+                           kTolAbs,
                            (unsigned long long*)doff.p, inner_sweeps);
       }
     }
@@ -1047,7 +1051,7 @@ int jacobi_svd_batched(Context& c, std::vector<JacobiBlock>& blocks, double tol,
   // hn holds the final column norms
   std::vector<int> ident(ncol);
   for (int b = 0; b < nb; ++b) {
-    JacobiBlock& J = blocks[b];
+    JacobiBlock& J = *blocks[b];
     const int k = K[b];
     // s_i = |W e_i| / |V e_i|: the singular value of the normalised triplet
     std::vector<double> s2(k);
@@ -1083,7 +1087,7 @@ int jacobi_svd_batched(Context& c, std::vector<JacobiBlock>& blocks, double tol,
   std::vector<PermJob> vj, wj;
   std::vector<VecMove> moves;
   for (int b = 0; b < nb; ++b) {
-    JacobiBlock& J = blocks[b];
+    JacobiBlock& J = *blocks[b];
     double* vdst = J.V == Vo[b] ? Vc[b] : J.V;
     vj.push_back(PermJob{Vo[b], vdst, K[b], K[b], 0, noff[b]});
     double* wdst = J.W == Wc[b] ? Wo[b] : J.W;
@@ -1111,6 +1115,21 @@ int jacobi_svd_batched(Context& c, std::vector<JacobiBlock>& blocks, double tol,
   // are already on the host
   SU2_HIP(hipGetLastError());
   return sweeps_done;
+}
+
+int jacobi_svd_batched(Context& c, std::vector<JacobiBlock>& blocks, double tol, int max_sweeps,
+                       int block_cols, int inner_sweeps, double* worst_out,
+                       int precondition_min_k) {
+  // a block's own shape decides, so its bits do not depend on the rest of
+  // the batch
+  std::vector<JacobiBlock*> small, large;
+  for (JacobiBlock& b : blocks) (small_svd_fits(b.m, b.n) ? small : large).push_back(&b);
+  double w1 = 0.0, w2 = 0.0;
+  const int n1 = small_svd_batched(c, small, tol, kTolAbs, kNoiseRel, max_sweeps, &w1);
+  const int n2 = jacobi_svd_large(c, large, tol, max_sweeps, block_cols, inner_sweeps, &w2,
+                                  precondition_min_k);
+  if (worst_out) *worst_out = std::max(w1, w2);
+  return std::max(n1, n2);
 }
 
 }  // namespace su2

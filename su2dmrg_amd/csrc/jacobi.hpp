@@ -10,6 +10,8 @@
 // the singular values, accurate relative to each value rather than to the
 // largest one.
 //
+// Blocks that fit one CU's LDS are decomposed there by one workgroup each
+// (small_svd.hpp); the rest of this description is about the larger ones.
 // Columns are cut into blocks of 16 (or 32).  A sweep visits every pair of blocks
 // once, in round-robin rounds of disjoint pairs; two kernel launches run all
 // pairs of a round for every block of the batch.  The first forms partial
