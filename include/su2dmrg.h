@@ -77,7 +77,7 @@ int su2_ctx_memory(su2_ctx* ctx, long long* live, long long* peak, long long* ca
  * visit of a pair 1..3 (default 1).  No counterpart in the reference; the
  * results agree to the SVD's own accuracy either way.  Blocks that fit one
  * compute unit's LDS (up to 96 x 96) are decomposed there, whatever is set
- * here or below. */
+ * here or below, unless nothing can be cut (su2_svd_truncate). */
 int su2_ctx_set_svd_tuning(su2_ctx* ctx, int block_cols, int inner_sweeps);
 /* QR preconditioning of the Jacobi SVD: for every sector block with
  * min_k <= min(m, n) <= 2048 (min_k 2..2048, default 256; 0 turns it off),
@@ -87,7 +87,8 @@ int su2_ctx_set_svd_tuning(su2_ctx* ctx, int block_cols, int inner_sweeps);
  * and a rank-deficient one (two-site wavefunction sectors typically are)
  * has its null directions in columns at the rounding level from the start,
  * which the sweeps leave out: a 16x8 D=2000 sweep takes about 26 s instead
- * of 37 s.
+ * of 37 s.  Blocks of fewer than 256 columns are always preconditioned, again
+ * unless nothing can be cut.
  * The reference computes its sector SVDs through the Gram matrix and dsyev
  * (tensor.cpp:1472-1529); this setting changes results by rounding only. */
 int su2_ctx_set_svd_precondition(su2_ctx* ctx, int min_k);
@@ -207,7 +208,11 @@ int su2_heff_set_kernel_path(su2_ctx* ctx, su2_heff* plan, int uniform, int* lay
  * s^p1, V = [psi leg 1, new bond] scaled by s^p2 (new tensors, destroy with
  * su2_tensor_destroy).  kept (nullable, capacity cap) receives the kept
  * singular values sector by sector, ascending within a sector; *nkept their
- * number; *discarded the summed squares of the cut values. */
+ * number; *discarded the summed squares of the cut values.  With max_dcut at
+ * least the columns of all sectors together nothing can be cut, and U and V
+ * hold every direction down to the rounding level: such a call uses the plain
+ * Jacobi iteration throughout (two to six times slower), so that those
+ * directions stay what they have been. */
 int su2_svd_truncate(su2_ctx* ctx, const su2_tensor* psi, double p1, double p2, int max_dcut,
                      su2_tensor** U, su2_tensor** V, double* kept, int cap, int* nkept,
                      double* discarded);

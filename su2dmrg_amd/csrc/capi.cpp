@@ -518,7 +518,7 @@ int su2_svd_truncate(su2_ctx* ctx, const su2_tensor* psi, double p1, double p2, 
     need(psi, "psi");
     need(U, "U");
     need(V, "V");
-    su2::SvdResult r = su2::truncated_svd(ctx->c, psi->t, p1, p2, max_dcut);
+    su2::SvdResult r = su2::truncated_svd(ctx->c, psi->t, p1, p2, max_dcut, true);
     int n = 0;
     for (auto& v : r.kept)
       for (double x : v) {

@@ -7,10 +7,12 @@
 #include <cstring>
 #include <memory>
 #include <numeric>
+#include <type_traits>
 
 #include "blas1.hpp"
 #include "common.hpp"
 #include "context.hpp"
+#include "ops.hpp"
 #include "precond.hpp"
 #include "small_svd.hpp"
 
@@ -18,7 +20,6 @@ namespace su2 {
 
 namespace {
 
-constexpr int RCH = 32;         // rows per staged chunk
 constexpr int INNER_SWEEPS = 3; // most inner Jacobi sweeps per visit of a pair
 constexpr int MAX_SLICES = 8;   // row slices per pair
 constexpr int MIN_SLICE_ROWS = 64;
@@ -26,9 +27,21 @@ constexpr int MIN_SLICE_ROWS = 64;
 // of the block: they carry no direction, no pair with one of them holds the
 // iteration open, and the sweeps leave them out of the schedule.
 constexpr double kNoiseRel = 1e-13;
+// Blocks under this many columns are preconditioned whatever the setting says:
+// a 192 x 192 block takes 5.5 ms that way and 14.4 ms without.
+constexpr int kPrecondAlways = 256;
+// Columns a first preconditioning pass left at or below this part of ||A||_F
+// (the square root of the pivot floor) are preconditioned again, if there are
+// at least kTailMin of them; there, pivots at or below kTailNoise ||A||_F are
+// the rounding of the first pass.
+constexpr double kTailRel = 3.2e-8;
+constexpr int kTailMin = 32;
+constexpr double kTailNoise = 3e-14;
 constexpr double kTolAbs = 1e-14;   // rounding floor of a pair, relative to ||A||_F
 
 typedef double f64x4 __attribute__((ext_vector_type(4)));
+typedef double f64x4u __attribute__((ext_vector_type(4), aligned(8)));   // any 8-byte address
+typedef double f64x2 __attribute__((ext_vector_type(2)));
 
 struct BlockDesc {
   double* W;        // L x k, ld L
@@ -41,12 +54,20 @@ struct PairJob {
   int blk;          // index into the block table
   int p0, bp;       // first column block
   int q0, bq;       // second column block (bq = 0: the first block alone)
-  int P;            // row slices (workgroups) that share the pair
+  int P;            // row slices (workgroups) that share the pair's Gram matrix
+  int full;         // rotate all its columns, not only those of p against q
 };
 
-__device__ __forceinline__ int rr_p(int r, int k, int m) { return k == 0 ? m - 1 : (r + k) % (m - 1); }
-__device__ __forceinline__ int rr_q(int r, int k, int m) {
-  return k == 0 ? r : (r - k + (m - 1)) % (m - 1);
+// Threads of the launches that diagonalise a pair and apply its rotations: one
+// wave that computes rotations and CB / 4 that apply them.
+template <int CB>
+struct SolveThreads {
+  static constexpr int value = 64 + 16 * CB;
+};
+
+// Column of W (or V) of a pair's column c.
+__device__ __forceinline__ int pair_column(const PairJob& J, int c) {
+  return c < J.bp ? J.p0 + c : J.q0 + (c - J.bp);
 }
 
 // 1 / x and 1 / sqrt(x) for x > 0 (normal): the hardware estimates
@@ -64,6 +85,19 @@ __device__ __forceinline__ double rsqrt_nr(double x) {
   return y * fma(-hx * y, y, 1.5);
 }
 
+// Scaled overlap of two columns from their Gram entries if it calls for a
+// rotation, else 0: relative orthogonality, or the rounding floor of columns
+// that carry absolute errors of order eps ||A||.  Columns at the rounding
+// level of the block carry no direction (the SVD zeroes them) and do not hold
+// the iteration open.
+__device__ __forceinline__ double pair_overlap(double gab, double ga, double gb, double tol_rel,
+                                               double tol_abs, double normF) {
+  const double g = fabs(gab), na = sqrt(ga), nb = sqrt(gb);
+  if (!(fmin(na, nb) > kNoiseRel * normF)) return 0.0;
+  const double scale = na * nb;
+  return g > fmax(tol_rel * scale, tol_abs * normF * (na + nb)) ? g / scale : 0.0;
+}
+
 // rows [lo, hi) of slice s when L rows are cut into P slices
 __device__ __forceinline__ void slice_rows(int L, int P, int s, int& lo, int& hi) {
   const int per = (L + P - 1) / P;
@@ -79,6 +113,15 @@ __device__ __forceinline__ void upper_tile(int u, int TT, int& tr, int& tc) {
     ++tr;
   }
   tc = tr + u;
+}
+
+// ---- the plain iteration's two launches per round ----
+
+constexpr int RCH = 32;         // rows per staged chunk
+
+__device__ __forceinline__ int rr_p(int r, int k, int m) { return k == 0 ? m - 1 : (r + k) % (m - 1); }
+__device__ __forceinline__ int rr_q(int r, int k, int m) {
+  return k == 0 ? r : (r - k + (m - 1)) % (m - 1);
 }
 
 // Partial Gram matrix of one pair over one row slice of W, on the matrix
@@ -510,6 +553,439 @@ __global__ __launch_bounds__(NT) void jacobi_rotate_kernel(const BlockDesc* __re
   }
 }
 
+// ---- the preconditioned iteration's launches ----
+
+// Pairs of column blocks that share one round, merged over the blocks of a batch: workgroups of a
+// launch find theirs by index.
+//
+// A visit of a pair takes three steps in as many launches (d = 2000 step, 34
+// pairs: 12, 37 and 20 us; the two launches of the plain iteration 15 and 93): partial Gram matrices over row slices
+// (gram_kernel), one workgroup per pair that sums them and diagonalises the pair's Gram matrix
+// (the first workgroups of solve_kernel), and the pair's columns times the rotation it found
+// (apply_rows), row tiles of W in a launch of their own.  V is not read before the sweep ends, so
+// its row tiles ride in the next round's solve launch, whose few workgroups leave the chip idle.
+
+// Partial Gram matrix of one pair over one row slice of W, on the matrix
+// cores.  The TT (TT + 1) / 2 tiles of 16 x 16 on and above the diagonal are
+// each a v_mfma_f64_16x16x4f64 chain over the rows: lane l holds rows 4 (l /
+// 16) .. + 3 of a 16-row strip in column l % 16 of each tile column (the same
+// assignment of rows to k for both operands, so any will do), which are 32
+// contiguous bytes: the loads go straight from memory to the fragments, with
+// no LDS pass and no barrier until the waves' sums meet.  Each wave takes
+// every fourth strip, the next strip's loads in flight under the MFMAs.  The
+// four partial sums are added in wave order; tile u's element of register q
+// and lane l goes to gpart[u][q][l].
+template <int CB>
+__global__ __launch_bounds__(256) void gram_kernel(const BlockDesc* __restrict__ blocks,
+                                                   const PairJob* __restrict__ jobs, int pmax,
+                                                   double* __restrict__ gpart) {
+  constexpr int NP = 2 * CB, TT = NP / 16, NU = TT * (TT + 1) / 2;
+  __shared__ double red[4][NU * 256];
+  const int job = blockIdx.x / pmax, slice = blockIdx.x - job * pmax;
+  const PairJob J = jobs[job];
+  if (slice >= J.P) return;
+  const BlockDesc B = blocks[J.blk];
+  const int n = J.bp + J.bq;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  int lo, hi;
+  slice_rows(B.L, J.P, slice, lo, hi);
+  const double* col[TT];
+  bool ok[TT];
+#pragma unroll
+  for (int i = 0; i < TT; ++i) {
+    const int c = 16 * i + (lane & 15);
+    ok[i] = c < n;
+    col[i] = B.W + (long long)pair_column(J, min(c, n - 1)) * B.L;
+  }
+  f64x4 acc[NU];
+#pragma unroll
+  for (int u = 0; u < NU; ++u) acc[u] = f64x4{0.0, 0.0, 0.0, 0.0};
+  f64x4 x[TT];
+  auto fetch = [&](int r0) {
+    const int r = r0 + 4 * (lane >> 4);
+    if (r0 + 16 <= hi) {
+#pragma unroll
+      for (int i = 0; i < TT; ++i) x[i] = *(const f64x4u*)(col[i] + r);
+    } else {
+#pragma unroll
+      for (int i = 0; i < TT; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) x[i][q] = r + q < hi ? col[i][r + q] : 0.0;
+    }
+#pragma unroll
+    for (int i = 0; i < TT; ++i)
+      if (!ok[i]) x[i] = f64x4{0.0, 0.0, 0.0, 0.0};
+  };
+  if (lo + 16 * wave < hi) fetch(lo + 16 * wave);
+  for (int r0 = lo + 16 * wave; r0 < hi; r0 += 64) {
+    f64x4 y[TT];
+#pragma unroll
+    for (int i = 0; i < TT; ++i) y[i] = x[i];
+    if (r0 + 64 < hi) fetch(r0 + 64);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      int u = 0;
+#pragma unroll
+      for (int a = 0; a < TT; ++a)
+#pragma unroll
+        for (int b = a; b < TT; ++b, ++u)
+          acc[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(y[a][q], y[b][q], acc[u], 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < NU; ++u)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) red[wave][256 * u + 64 * q + lane] = acc[u][q];
+  __syncthreads();
+  double* out = gpart + (size_t)blockIdx.x * NU * 256;
+  for (int e = t; e < NU * 256; e += 256)
+    out[e] = ((red[0][e] + red[1][e]) + red[2][e]) + red[3][e];
+}
+
+// LDS of one pair: G (upper triangle) and R[column][row], both NP x NP, cos
+// and sin and tan of each slot (two buffers), whether a sweep rotated.
+struct PairLds {
+  double* G;
+  double* R;
+  f64x2* cs;
+  double* tn;
+  int* rotated;
+};
+
+// The inner sweeps of one pair of n columns; FULL: all of them against each
+// other, else the first CB against the others.
+template <int CB, bool FULL>
+__device__ __forceinline__ void pair_sweeps(const PairLds& S, int n, double fl,
+                                            int inner_sweeps) {
+  constexpr int NP = 2 * CB, NT = SolveThreads<CB>::value;
+  double* G = S.G;
+  double* R = S.R;
+  f64x2* cs = S.cs;
+  double* tn = S.tn;
+  int* rotated = S.rotated;
+  const int t = threadIdx.x;
+  const int m = n + (n & 1);   // index n (odd n) is a zero row and column
+  const int nround = FULL ? m - 1 : CB;
+  const double tol_in = 1e-14;
+  // columns of slot k in round r: the round-robin pair in a full sweep
+  // (identity slots (2k, 2k+1) past the last pair), else k and a q column
+  auto slot = [&](int r, int k, int& p, int& q) {
+    if (!FULL) {
+      p = k;
+      q = CB + ((k + r) & (CB - 1));
+    } else if (k < m / 2) {
+      p = k == 0 ? m - 1 : (r + k < m - 1 ? r + k : r + k - (m - 1));
+      q = k == 0 ? r : (r >= k ? r - k : r - k + (m - 1));
+    } else {
+      p = 2 * k;
+      q = 2 * k + 1;
+    }
+  };
+  auto at = [&](int a, int b) { return min(a, b) * NP + max(a, b); };
+  auto rotation = [&](int r, int k, int b, int sweep) {
+    int p, q;
+    slot(r, k, p, q);
+    double c = 1.0, s = 0.0, tt = 0.0;
+    if (p < n && q < n) {
+      const double apq = G[at(p, q)], gpp = G[p * NP + p], gqq = G[q * NP + q];
+      const double app = fabs(gpp), aqq = fabs(gqq), a2 = apq * apq;
+      if (a2 > tol_in * tol_in * (app * aqq) && a2 > 4.0 * fl * fl * fmax(app, aqq) &&
+          fabs(apq) > 1e-300) {
+        // t = tan(theta) of the smaller rotation angle,
+        //   t = 2 g_pq sign(d) / (|d| + sqrt(d^2 + 4 g_pq^2)), d = g_qq - g_pp;
+        // c = 1 / sqrt(1 + t^2) keeps the rotation orthogonal to rounding for
+        // any t, so the reciprocals need not be correctly rounded
+        const double d = gqq - gpp, h2 = d * d + 4.0 * a2;
+        const double den = fabs(d) + h2 * rsqrt_nr(h2);
+        tt = (d >= 0 ? 2.0 : -2.0) * apq * recip_nr(den);
+        c = rsqrt_nr(1.0 + tt * tt);
+        s = tt * c;
+        rotated[sweep] = 1;
+      }
+    }
+    cs[b * CB + k] = f64x2{c, s};
+    tn[b * CB + k] = tt;
+  };
+  // the 2 x 2 block of slots k and k2; a slot's own block (k == k2) has its
+  // entry annihilated exactly and its diagonal moved by t g_pq
+  auto mix = [&](int r, int b, int k, int k2) {
+    int p, q, p2, q2;
+    slot(r, k, p, q);
+    slot(r, k2, p2, q2);
+    const int e00 = at(p, p2), e01 = at(p, q2), e10 = at(q, p2), e11 = at(q, q2);
+    const double g00 = G[e00], g01 = G[e01], g10 = G[e10], g11 = G[e11];
+    const f64x2 x = cs[b * CB + k], y = cs[b * CB + k2];
+    const double tt = tn[b * CB + k];
+    const double t00 = y.x * g00 - y.y * g01, t01 = y.y * g00 + y.x * g01;
+    const double t10 = y.x * g10 - y.y * g11, t11 = y.y * g10 + y.x * g11;
+    const bool own = k == k2, hit = own && tt != 0.0;
+    const double n01 = x.x * t01 - x.y * t11, n10 = x.y * t00 + x.x * t10;
+    G[e00] = own ? g00 - tt * g01 : x.x * t00 - x.y * t10;
+    G[e11] = own ? g11 + tt * g01 : x.y * t01 + x.x * t11;
+    G[e01] = hit ? 0.0 : n01;
+    G[e10] = hit ? 0.0 : own ? n01 : n10;
+  };
+  // G: threads (k, d), d = 1 .. CB/2 - 1, take slots k and k + d modulo CB;
+  // then CB threads a slot's own block and CB / 2 the slots CB / 2 apart
+  const int k = t % CB, d = t / CB + 1;
+  constexpr int D = CB / 2;
+  static_assert(CB * D + D <= NT, "threads of the G update");
+  const int k2 = d < D ? (k + d) % CB : d == D ? k : (k + D) % CB;
+  const bool mine = d <= D || (d == D + 1 && k < D);
+  // R: four slots' elements of one row per thread.  In cross rounds a slot's
+  // p column is always the same, so its element stays in a register.
+  constexpr int NR = NT - 64, SL = CB * NP / NR;
+  static_assert(SL * NR == CB * NP && NR % NP == 0, "slots per thread");
+  const int row = (t - 64) % NP, k0 = (t - 64) / NP;
+  double u[SL];
+  if (!FULL && t >= 64) {
+#pragma unroll
+    for (int i = 0; i < SL; ++i) u[i] = R[(k0 + i * (NR / NP)) * NP + row];
+  }
+  if (t < CB) rotation(0, t, 0, 0);
+  __syncthreads();
+  int b = 0;
+  for (int sweep = 0; sweep < inner_sweeps; ++sweep) {
+    for (int r = 0; r < nround; ++r, b ^= 1) {
+      if (mine) mix(r, b, k, k2);
+      __syncthreads();
+      const bool last = r + 1 == nround;
+      const int sw = last ? sweep + 1 : sweep;
+      if (t < 64) {
+        if (t < CB && sw < inner_sweeps) rotation(last ? 0 : r + 1, t, b ^ 1, sw);
+      } else {
+        // R <- R J, all loads before the first store
+        double v[SL];
+        f64x2 x[SL];
+        int p[SL], q[SL];
+#pragma unroll
+        for (int i = 0; i < SL; ++i) {
+          const int kk = k0 + i * (NR / NP);
+          x[i] = cs[b * CB + kk];
+          slot(r, kk, p[i], q[i]);
+          if (FULL) u[i] = R[p[i] * NP + row];
+          v[i] = R[q[i] * NP + row];
+        }
+#pragma unroll
+        for (int i = 0; i < SL; ++i) {
+          const double w = x[i].x * u[i] - x[i].y * v[i];
+          R[q[i] * NP + row] = x[i].y * u[i] + x[i].x * v[i];
+          u[i] = w;
+          if (FULL) R[p[i] * NP + row] = w;
+        }
+      }
+      __syncthreads();
+    }
+    if (!rotated[sweep]) break;
+  }
+  if (!FULL && t >= 64) {
+#pragma unroll
+    for (int i = 0; i < SL; ++i) R[(k0 + i * (NR / NP)) * NP + row] = u[i];
+  }
+  __syncthreads();
+}
+
+// Diagonalises one pair's Gram matrix: the slices' partial sums in slice
+// order, the convergence test, then inner_sweeps sweeps of parallel cyclic
+// Jacobi in LDS, and the accumulated rotation to rot (column-major, NP rows).
+// *active says whether the pair rotated at all.
+//
+// A pair rotates its p columns against its q columns only (CB rounds of CB
+// disjoint rotations): the pairs inside a block are rotated in the block's
+// first visit of a sweep (J.full: 2 CB - 1 rounds over all its columns), so a
+// sweep meets every pair of columns once.  A model of the iteration at k =
+// 640 needed 908 such visits against 886 that rotate all pairs every time,
+// each at half the rounds.
+//
+// G is symmetric, and only its upper triangle is kept: the rotations of slots
+// k and k2 mix four elements, one thread's, at distinct places.  A round is
+// two phases with a barrier each: every thread updates its 2 x 2 block (its
+// LDS reads do not wait for the rotations' parameters); then wave 0 computes
+// the next round's rotations while the other waves apply this round's to R
+// (double-buffered parameters).  In cross rounds neighbouring threads' blocks
+// lie NP + 1 apart, which spreads them over all LDS banks at a pitch of NP.
+// Clock stamps of a cross round: 600 cycles of G, 1000 of R beside 700 of the
+// rotations (2600 with the barriers; the plain launch takes 2900 for half the
+// work of a round, being one group of threads after another).
+// A rotation annihilates its entry exactly and moves the diagonal by t g_pq;
+// it is skipped below max(tol_in sqrt(g_pp g_qq), 0.2 tol_abs ||A||_F
+// sqrt(max(g_pp, g_qq))), about ten times below the outer test.
+template <int CB>
+__device__ __forceinline__ void solve_pair(const BlockDesc& B, const PairJob& J,
+                                           const double* __restrict__ gp, double tol_rel,
+                                           double tol_abs, int inner_sweeps, double* lds,
+                                           double* __restrict__ rot, int* __restrict__ active) {
+  constexpr int NP = 2 * CB, TT = NP / 16, NU = TT * (TT + 1) / 2, NT = SolveThreads<CB>::value;
+  double* G = lds;                       // NP x NP, upper triangle
+  double* R = G + NP * NP;               // R[column][row]
+  f64x2* cs = (f64x2*)(R + NP * NP);     // cos, sin of slot k: [2][CB]
+  double* tn = (double*)(cs + 2 * CB);   // tan: [2][CB]
+  int* rotated = (int*)(tn + 2 * CB);    // INNER_SWEEPS
+  const int n = J.bp + J.bq, t = threadIdx.x;
+  if (t < INNER_SWEEPS) rotated[t] = 0;
+  for (int e = t; e < NP * NP; e += NT) R[e] = e / NP == e % NP ? 1.0 : 0.0;
+  {
+    // the slices' sums; all loads of a thread are in flight at once
+    constexpr int PER = (NU * 256 + NT - 1) / NT;
+    double part[PER][MAX_SLICES];
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+#pragma unroll
+      for (int s = 0; s < MAX_SLICES; ++s)
+        part[i][s] = s < J.P ? gp[(size_t)s * NU * 256 + min(t + NT * i, NU * 256 - 1)] : 0.0;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int e = t + NT * i;
+      if (e >= NU * 256) break;
+      double g = 0.0;
+#pragma unroll
+      for (int s = 0; s < MAX_SLICES; ++s)
+        if (s < J.P) g += part[i][s];
+      int tr, tc;
+      upper_tile(e / 256, TT, tr, tc);
+      const int l = e & 63, q = (e >> 6) & 3;
+      G[(16 * tr + (l >> 4) + 4 * q) * NP + 16 * tc + (l & 15)] = g;
+    }
+  }
+  __syncthreads();
+
+  // ---- does the pair need a rotation? ----
+  double* norm = tn;   // free until the rotations
+  if (t < n) norm[t] = sqrt(G[t * NP + t]);
+  __syncthreads();
+  bool need = false;
+  {
+    const double noise = kNoiseRel * B.normF, ta = tol_abs * B.normF;
+    const int ra = J.full ? n : J.bp;   // rows a of the entries looked at
+    for (int e = t; e < ra * NP; e += NT) {
+      const int a = e / NP, b = e % NP;
+      if (b >= n || b <= a || (!J.full && b < J.bp)) continue;
+      const double na = norm[a], nb = norm[b];
+      need = need || (fmin(na, nb) > noise &&
+                      fabs(G[a * NP + b]) > fmax(tol_rel * na * nb, ta * (na + nb)));
+    }
+  }
+  const bool any = __syncthreads_or(need);
+  if (t == 0) *active = any;
+  if (!any) return;
+
+  PairLds L{G, R, cs, tn, rotated};
+  const double fl = 0.1 * tol_abs * B.normF;
+  if (J.full) pair_sweeps<CB, true>(L, n, fl, inner_sweeps);
+  else pair_sweeps<CB, false>(L, n, fl, inner_sweeps);
+  for (int e = t; e < NP * NP; e += NT) rot[e] = R[e];
+}
+
+// M[rows, cols] <- M[rows, cols] R for one row tile of W or V, 16 rows per wave.  R goes to LDS; a wave's 16 x NP strip goes straight from
+// memory to its B fragments (lane l: row l % 16, column 4 s + l / 16, 128
+// contiguous bytes per column), and Y^T = R^T X^T comes back with 16 rows of
+// a column on neighbouring lanes, so it is stored as it is.  A wave owns its
+// rows and reads them before it writes, so the update is in place.
+template <int CB>
+__device__ __forceinline__ void apply_rows(double* __restrict__ M, int rows, const PairJob& J,
+                                           const double* __restrict__ rot, int tile,
+                                           double* lds) {
+  constexpr int NP = 2 * CB, TT = NP / 16, NT = SolveThreads<CB>::value, PR = NP + 1;
+  const int n = J.bp + J.bq, t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int r0 = tile * (NT / 4) + wave * 16;
+  const int row = min(r0 + (lane & 15), rows - 1);
+  double x[NP / 4];
+#pragma unroll
+  for (int s = 0; s < NP / 4; ++s) {
+    const int c = 4 * s + (lane >> 4);
+    x[s] = M[row + (long long)pair_column(J, min(c, n - 1)) * rows];
+  }
+  for (int e = t; e < NP * NP; e += NT) lds[(e % NP) * PR + e / NP] = rot[e];
+  __syncthreads();
+#pragma unroll
+  for (int s = 0; s < NP / 4; ++s)
+    if (4 * s + (lane >> 4) >= n) x[s] = 0.0;
+  f64x4 y[TT];
+#pragma unroll
+  for (int i = 0; i < TT; ++i) y[i] = f64x4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int s = 0; s < NP / 4; ++s)
+#pragma unroll
+    for (int i = 0; i < TT; ++i)
+      y[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+          lds[(4 * s + (lane >> 4)) * PR + 16 * i + (lane & 15)], x[s], y[i], 0, 0, 0);
+  if (r0 + (lane & 15) >= rows) return;
+#pragma unroll
+  for (int i = 0; i < TT; ++i)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int c = 16 * i + (lane >> 4) + 4 * q;
+      if (c < n) M[row + (long long)pair_column(J, c) * rows] = y[i][q];
+    }
+}
+
+// The first nj workgroups diagonalise this round's pairs, the others apply
+// the previous round's rotations to V's row tiles (nv of them per pair).
+template <int CB>
+__global__ __launch_bounds__(SolveThreads<CB>::value) void solve_kernel(
+    const BlockDesc* __restrict__ blocks, const PairJob* __restrict__ jobs, int nj, int pmax,
+    const double* __restrict__ gpart, double tol_rel, double tol_abs, int inner_sweeps,
+    double* __restrict__ rot, int* __restrict__ active, const PairJob* __restrict__ vjobs, int nv,
+    const double* __restrict__ vrot, const int* __restrict__ vactive) {
+  constexpr int NP = 2 * CB, NU = (NP / 16) * (NP / 16 + 1) / 2;
+  __shared__ __align__(16) double lds[2 * NP * NP + 6 * CB + 2];
+  const int i = blockIdx.x;
+  if (i < nj) {
+    const PairJob J = jobs[i];
+    solve_pair<CB>(blocks[J.blk], J, gpart + (size_t)i * pmax * NU * 256, tol_rel, tol_abs,
+                   inner_sweeps, lds, rot + (size_t)i * NP * NP, active + i);
+    return;
+  }
+  const int job = (i - nj) / nv, tile = (i - nj) - job * nv;
+  const PairJob J = vjobs[job];
+  const BlockDesc B = blocks[J.blk];
+  if (tile * (SolveThreads<CB>::value / 4) >= B.k || !vactive[job]) return;
+  apply_rows<CB>(B.V, B.k, J, vrot + (size_t)job * NP * NP, tile, lds);
+}
+
+// This round's rotations on W's row tiles (ntile per pair).
+template <int CB>
+__global__ __launch_bounds__(SolveThreads<CB>::value) void apply_kernel(
+    const BlockDesc* __restrict__ blocks, const PairJob* __restrict__ jobs, int ntile,
+    const double* __restrict__ rot, const int* __restrict__ active) {
+  constexpr int NP = 2 * CB;
+  __shared__ double lds[NP * (NP + 1)];
+  const int job = blockIdx.x / ntile, tile = blockIdx.x - job * ntile;
+  const PairJob J = jobs[job];
+  const BlockDesc B = blocks[J.blk];
+  if (tile * (SolveThreads<CB>::value / 4) >= B.L || !active[job]) return;
+  apply_rows<CB>(B.W, B.L, J, rot + (size_t)job * NP * NP, tile, lds);
+}
+
+// Largest overlap that calls for a rotation in each pair of column blocks (i
+// <= j) of a block's kept columns, from their whole Gram matrix (0: none);
+// workgroup = entry of the pair table.
+struct FlagJob {
+  const double* G;   // kept x kept, ld ldg
+  int ldg, kept, i, j;
+  double normF;
+};
+
+__global__ __launch_bounds__(256) void pair_flags_kernel(const FlagJob* __restrict__ jobs, int cb,
+                                                         double tol_rel, double tol_abs,
+                                                         double* __restrict__ out) {
+  __shared__ double s[4];
+  const FlagJob J = jobs[blockIdx.x];
+  double worst = 0.0;
+  for (int e = threadIdx.x; e < cb * cb; e += 256) {
+    const int a = J.i * cb + e % cb, b = J.j * cb + e / cb;
+    if (a >= b || b >= J.kept) continue;
+    const double ga = J.G[a + (size_t)a * J.ldg], gb = J.G[b + (size_t)b * J.ldg];
+    worst = fmax(worst, pair_overlap(J.G[a + (size_t)b * J.ldg], ga, gb, tol_rel, tol_abs,
+                                     J.normF));
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) worst = fmax(worst, __shfl_xor(worst, o));
+  if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = worst;
+  __syncthreads();
+  if (threadIdx.x == 0) out[blockIdx.x] = fmax(fmax(s[0], s[1]), fmax(s[2], s[3]));
+}
+
 // W = A (transpose = 0) or A^T (transpose = 1); A is m x n with ld m
 __global__ void load_work_kernel(const double* __restrict__ A, int m, int n, int transpose,
                                  double* __restrict__ W) {
@@ -731,7 +1207,7 @@ struct DevMem {
 
 static int jacobi_svd_large(Context& c, const std::vector<JacobiBlock*>& blocks, double tol,
                             int max_sweeps, int block_cols, int inner_sweeps, double* worst_out,
-                            int precondition_min_k) {
+                            int precondition_min_k, bool plain) {
   if (worst_out) *worst_out = 0.0;
   hipStream_t st = c.stream();
   const int nb = (int)blocks.size();
@@ -832,12 +1308,20 @@ static int jacobi_svd_large(Context& c, const std::vector<JacobiBlock*>& blocks,
   std::vector<char> active(nb, 1);
   auto sort_permute = [&]() {
     std::vector<PermJob> pj;
+    std::vector<char> moved(nb, 0);
     for (int b = 0; b < nb; ++b) {
       if (!active[b]) continue;
       int* p = hp.data() + noff[b];
       const double* w = hn.data() + noff[b];
       std::iota(p, p + K[b], 0);
       std::stable_sort(p, p + K[b], [&](int x, int y) { return w[x] > w[y]; });
+      moved[b] = !std::is_sorted(p, p + K[b]);
+      if (!moved[b]) continue;
+      // the norms follow their columns
+      for (long long h : {noff[b], ncol + noff[b]}) {
+        std::vector<double> old(hn.begin() + h, hn.begin() + h + K[b]);
+        for (int i = 0; i < K[b]; ++i) hn[h + i] = old[p[i]];
+      }
       pj.push_back(PermJob{Wc[b], Wo[b], L[b], K[b], 0, noff[b]});
       pj.push_back(PermJob{Vc[b], Vo[b], K[b], K[b], 0, noff[b]});
     }
@@ -845,7 +1329,7 @@ static int jacobi_svd_large(Context& c, const std::vector<JacobiBlock*>& blocks,
     SU2_HIP(hipMemcpyAsync(dperm.p, hp.data(), sizeof(int) * ncol, hipMemcpyHostToDevice, st));
     permute(pj, (const double*)done.p);
     for (int b = 0; b < nb; ++b) {
-      if (!active[b]) continue;
+      if (!moved[b]) continue;
       std::swap(Wc[b], Wo[b]);
       std::swap(Vc[b], Vo[b]);
     }
@@ -856,15 +1340,18 @@ static int jacobi_svd_large(Context& c, const std::vector<JacobiBlock*>& blocks,
   // own size decides, so its bits do not depend on the rest of the batch (a
   // block left out is sorted here instead of at the first sweep: the same
   // permutation, and the first sweep's sort is then the identity).
-  if (precondition_min_k > 0) {
+  {
     std::vector<PrecondBlock> pb;
     std::vector<int> pre;
     for (int b = 0; b < nb; ++b)
-      if (K[b] >= precondition_min_k && K[b] <= kPrecondMaxK) pre.push_back(b);
+      if ((!plain && K[b] < kPrecondAlways) ||
+          (precondition_min_k > 0 && K[b] >= precondition_min_k && K[b] <= kPrecondMaxK)) {
+        pre.push_back(b);
+      }
     if (!pre.empty()) {
       sort_permute();
       for (int b : pre)
-        pb.push_back(PrecondBlock{Wc[b], Vc[b], Wo[b], Vo[b], L[b], K[b], desc[b].normF});
+        pb.push_back(PrecondBlock{Wc[b], Vc[b], Wo[b], Vo[b], L[b], K[b], K[b], desc[b].normF, 0.0});
       precondition_jacobi(c, pb);
       for (int b : pre) {
         std::swap(Wc[b], Wo[b]);
@@ -872,6 +1359,43 @@ static int jacobi_svd_large(Context& c, const std::vector<JacobiBlock*>& blocks,
       }
       upload_desc();
       norms();
+      // The Gram matrix resolves directions down to 3e-8 of the block; the
+      // columns below that are still a mixture of everything under it.
+      // They are preconditioned among themselves, with their own Gram matrix
+      // (which resolves 3e-8 of theirs), so that the null space drops to the
+      // rounding level at once and leaves the sweeps.
+      if (!plain) sort_permute();
+      std::vector<PrecondBlock> tail;
+      std::vector<VecMove> back;
+      for (const int b : plain ? std::vector<int>() : pre) {
+        const double thr = kTailRel * desc[b].normF * (kTailRel * desc[b].normF);
+        int r = 0;
+        while (r < K[b] && hn[noff[b] + r] > thr) ++r;
+        const int n = K[b] - r;
+        if (n < kTailMin) continue;
+        double top = 0.0, sum = 0.0;
+        for (int q = r; q < K[b]; ++q) {
+          const double w = hn[noff[b] + q];
+          top = std::max(top, w);
+          sum += w;
+        }
+        if (!(std::sqrt(top) > kNoiseRel * desc[b].normF)) continue;
+        const long long wo = (long long)r * L[b], vo = (long long)r * K[b];
+        tail.push_back(PrecondBlock{Wc[b] + wo, Vc[b] + vo, Wo[b] + wo, Vo[b] + vo, L[b], n, K[b],
+                                    std::sqrt(sum), kTailNoise * desc[b].normF});
+        back.push_back(VecMove{Wo[b] + wo, Wc[b] + wo, (long long)n * L[b], kMoveF64, 0});
+        back.push_back(VecMove{Vo[b] + vo, Vc[b] + vo, (long long)n * K[b], kMoveF64, 0});
+      }
+      if (!tail.empty()) {
+        precondition_jacobi(c, tail);
+        long long mx = 0;
+        for (auto& m : back) mx = std::max(mx, m.n);
+        DevMem dm(c, sizeof(VecMove) * back.size());
+        SU2_HIP(hipMemcpyAsync(dm.p, back.data(), sizeof(VecMove) * back.size(),
+                               hipMemcpyHostToDevice, st));
+        dev_move_batch(c, (const VecMove*)dm.p, (int)back.size(), mx);
+      }
+      if (!tail.empty()) norms();
     }
   }
   // Deflation: the columns of a block above the rounding level, kept[b] of
@@ -895,49 +1419,24 @@ static int jacobi_svd_large(Context& c, const std::vector<JacobiBlock*>& blocks,
     return changed;
   };
   count_kept();
-  // round-robin schedule of column-block pairs of the active blocks' kept
-  // columns, merged across blocks by round
+  // the pairs of a sweep by round, and their launch order
   std::vector<std::vector<PairJob>> rounds;
   std::vector<int> round_off, round_pmax;
   std::vector<PairJob> all;
-  size_t gpart_max = 0;
-  auto build_schedule = [&]() {
-    rounds.clear();
+  auto slice_rounds = [&]() {
     all.clear();
-    gpart_max = 0;
-    for (int b = 0; b < nb; ++b) {
-      if (!active[b]) continue;
-      const int kb = kept[b];
-      const int ncb = (kb + CB - 1) / CB;
-      auto width = [&](int i) { return i >= ncb ? 0 : std::min(CB, kb - i * CB); };
-      if (ncb <= 1) {
-        if (rounds.empty()) rounds.resize(1);
-        if (kb >= 2) rounds[0].push_back(PairJob{b, 0, kb, 0, 0, 1});
-        continue;
-      }
-      const int mp = ncb + (ncb & 1);
-      if ((int)rounds.size() < mp - 1) rounds.resize(mp - 1);
-      for (int r = 0; r < mp - 1; ++r)
-        for (int k = 0; k < mp / 2; ++k) {
-          int P = (k == 0) ? mp - 1 : (r + k) % (mp - 1);
-          int Q = (k == 0) ? r : (r - k + (mp - 1)) % (mp - 1);
-          if (width(P) == 0) std::swap(P, Q);
-          if (width(P) == 0) continue;
-          rounds[r].push_back(PairJob{b, P * CB, width(P), width(Q) ? Q * CB : 0, width(Q), 1});
-        }
-    }
     // Row slices: a group (the sectors of one wavefunction) with few pairs in
-    // a round spreads each pair over up to MAX_SLICES workgroups (at least 64
-    // rows each), about slice_target workgroups per group and round, so that
-    // the round fills the chip.  The slice count of a pair follows from its own
-    // group alone, never from the other groups of the batch: the slices'
-    // partial Gram matrices are summed in slice order, so the slicing decides
-    // the bits, and a wavefunction gets the same bits alone and in a batch.
+    // a round spreads each pair's Gram matrix over up to MAX_SLICES workgroups
+    // (at least 64 rows each), about slice_target workgroups per group and
+    // round, so that the round fills the chip.  The slice count of a pair
+    // follows from its own group alone, never from the other groups of the
+    // batch: the slices' partial Gram matrices are summed in slice order, so
+    // the slicing decides the bits, and a wavefunction gets the same bits
+    // alone and in a batch.
     round_off.assign(rounds.size() + 1, 0);
     round_pmax.assign(rounds.size(), 1);
     for (size_t r = 0; r < rounds.size(); ++r) {
       round_off[r] = (int)all.size();
-      const int nj = (int)rounds[r].size();
       std::map<int, int> per_group;
       for (const PairJob& j : rounds[r]) per_group[blocks[j.blk]->group]++;
       int used = 1;
@@ -948,92 +1447,300 @@ static int jacobi_svd_large(Context& c, const std::vector<JacobiBlock*>& blocks,
         used = std::max(used, j.P);
       }
       round_pmax[r] = used;
-      gpart_max = std::max(gpart_max, (size_t)nj * used);
       all.insert(all.end(), rounds[r].begin(), rounds[r].end());
     }
     round_off[rounds.size()] = (int)all.size();
   };
-  // the full schedule sizes the buffers; a smaller one replaces it in place
-  // (a pair of a smaller schedule may take more slices, never more than
-  // MAX_SLICES, and no round has more pairs than the full one's)
-  build_schedule();
-  size_t gpart_cap = 1;
-  for (size_t r = 0; r + 1 < round_off.size(); ++r)
-    gpart_cap = std::max(gpart_cap, (size_t)(round_off[r + 1] - round_off[r]) * MAX_SLICES);
-  DevMem dgpart(c, sizeof(double) * NP * NP * gpart_cap);
-  DevMem djobs(c, sizeof(PairJob) * std::max<size_t>(1, all.size())),
-      doff(c, sizeof(unsigned long long) * nb);
-  auto upload_jobs = [&]() {
-    if (!all.empty())
-      SU2_HIP(hipMemcpyAsync(djobs.p, all.data(), sizeof(PairJob) * all.size(),
-                             hipMemcpyHostToDevice, st));
-  };
-  upload_jobs();
-  std::vector<unsigned long long> hoff(nb);
-  bool converged = all.empty();
+  bool converged = false;
   double worst = 0;
   int sweeps_done = 0;
-  for (int sweep = 0; sweep < max_sweeps && !converged; ++sweep) {
-    ++sweeps_done;
-    // descending column norms (hn: read back with the previous sweep's
-    // convergence counters, or before the first sweep)
-    sort_permute();
-    hipLaunchKernelGGL(fill_u64_kernel, dim3(nblk(nb, 256)), dim3(256), 0, st,
-                       (unsigned long long*)doff.p, nb);
-    for (size_t r = 0; r < rounds.size(); ++r) {
-      const int nj = round_off[r + 1] - round_off[r];
-      if (nj == 0) continue;
-      const int pm = round_pmax[r];
-      const PairJob* jr = (const PairJob*)djobs.p + round_off[r];
-      if (CB == 16) {
-        hipLaunchKernelGGL((gram_partial_kernel<16, 64, RCH>), dim3(nj * pm), dim3(64), 0, st,
-                           (const BlockDesc*)ddesc.p, jr, pm, (double*)dgpart.p);
-        hipLaunchKernelGGL((jacobi_rotate_kernel<16, 64>), dim3(nj * pm), dim3(64), 0, st,
-                           (const BlockDesc*)ddesc.p, jr, pm, (const double*)dgpart.p, tol,
-                           kTolAbs,
-                           (unsigned long long*)doff.p, inner_sweeps);
-      } else {
-        hipLaunchKernelGGL((gram_partial_kernel<32, 1024, 64>), dim3(nj * pm), dim3(1024), 0, st,
-                           (const BlockDesc*)ddesc.p, jr, pm, (double*)dgpart.p);
-        hipLaunchKernelGGL((jacobi_rotate_kernel<32, 512>), dim3(nj * pm), dim3(512), 0, st,
-                           (const BlockDesc*)ddesc.p, jr, pm, (const double*)dgpart.p, tol,
-                           kTolAbs,
-                           (unsigned long long*)doff.p, inner_sweeps);
+  if (plain) {
+    // round-robin schedule of column-block pairs of the active blocks' kept
+    // columns, merged across blocks by round
+    auto build_schedule = [&]() {
+      rounds.clear();
+      all.clear();
+      for (int b = 0; b < nb; ++b) {
+        if (!active[b]) continue;
+        const int kb = kept[b];
+        const int ncb = (kb + CB - 1) / CB;
+        auto width = [&](int i) { return i >= ncb ? 0 : std::min(CB, kb - i * CB); };
+        if (ncb <= 1) {
+          if (rounds.empty()) rounds.resize(1);
+          if (kb >= 2) rounds[0].push_back(PairJob{b, 0, kb, 0, 0, 1, 0});
+          continue;
+        }
+        const int mp = ncb + (ncb & 1);
+        if ((int)rounds.size() < mp - 1) rounds.resize(mp - 1);
+        for (int r = 0; r < mp - 1; ++r)
+          for (int k = 0; k < mp / 2; ++k) {
+            int P = (k == 0) ? mp - 1 : (r + k) % (mp - 1);
+            int Q = (k == 0) ? r : (r - k + (mp - 1)) % (mp - 1);
+            if (width(P) == 0) std::swap(P, Q);
+            if (width(P) == 0) continue;
+            rounds[r].push_back(PairJob{b, P * CB, width(P), width(Q) ? Q * CB : 0, width(Q), 1, 0});
+          }
+      }
+      slice_rounds();
+    };
+    // the full schedule sizes the buffers; a smaller one replaces it in place
+    // (a pair of a smaller schedule may take more slices, never more than
+    // MAX_SLICES, and no round has more pairs than the full one's)
+    build_schedule();
+    size_t gpart_cap = 1;
+    for (size_t r = 0; r + 1 < round_off.size(); ++r)
+      gpart_cap = std::max(gpart_cap, (size_t)(round_off[r + 1] - round_off[r]) * MAX_SLICES);
+    DevMem dgpart(c, sizeof(double) * NP * NP * gpart_cap);
+    DevMem djobs(c, sizeof(PairJob) * std::max<size_t>(1, all.size())),
+        doff(c, sizeof(unsigned long long) * nb);
+    auto upload_jobs = [&]() {
+      if (!all.empty())
+        SU2_HIP(hipMemcpyAsync(djobs.p, all.data(), sizeof(PairJob) * all.size(),
+                               hipMemcpyHostToDevice, st));
+    };
+    upload_jobs();
+    std::vector<unsigned long long> hoff(nb);
+    converged = all.empty();
+    for (int sweep = 0; sweep < max_sweeps && !converged; ++sweep) {
+      ++sweeps_done;
+      // descending column norms (hn: read back with the previous sweep's
+      // convergence counters, or before the first sweep)
+      sort_permute();
+      hipLaunchKernelGGL(fill_u64_kernel, dim3(nblk(nb, 256)), dim3(256), 0, st,
+                         (unsigned long long*)doff.p, nb);
+      for (size_t r = 0; r < rounds.size(); ++r) {
+        const int nj = round_off[r + 1] - round_off[r];
+        if (nj == 0) continue;
+        const int pm = round_pmax[r];
+        const PairJob* jr = (const PairJob*)djobs.p + round_off[r];
+        if (CB == 16) {
+          hipLaunchKernelGGL((gram_partial_kernel<16, 64, RCH>), dim3(nj * pm), dim3(64), 0, st,
+                             (const BlockDesc*)ddesc.p, jr, pm, (double*)dgpart.p);
+          hipLaunchKernelGGL((jacobi_rotate_kernel<16, 64>), dim3(nj * pm), dim3(64), 0, st,
+                             (const BlockDesc*)ddesc.p, jr, pm, (const double*)dgpart.p, tol,
+                             kTolAbs,
+                             (unsigned long long*)doff.p, inner_sweeps);
+        } else {
+          hipLaunchKernelGGL((gram_partial_kernel<32, 1024, 64>), dim3(nj * pm), dim3(1024), 0, st,
+                             (const BlockDesc*)ddesc.p, jr, pm, (double*)dgpart.p);
+          hipLaunchKernelGGL((jacobi_rotate_kernel<32, 512>), dim3(nj * pm), dim3(512), 0, st,
+                             (const BlockDesc*)ddesc.p, jr, pm, (const double*)dgpart.p, tol,
+                             kTolAbs,
+                             (unsigned long long*)doff.p, inner_sweeps);
+        }
+      }
+      SU2_HIP(hipGetLastError());
+      SU2_HIP(hipMemcpyAsync(hoff.data(), doff.p, sizeof(unsigned long long) * nb,
+                             hipMemcpyDeviceToHost, st));
+      // the column norms for the next sweep's order (or the final one) come
+      // back with the counters: one wait per sweep
+      hipLaunchKernelGGL(colnorm_batched_kernel, dim3((unsigned)ncol), dim3(256), 0, st,
+                         (const BlockDesc*)ddesc.p, (const long long*)dnoff.p, nb, (long long)ncol,
+                         (double*)dn.p);
+      SU2_HIP(hipMemcpyAsync(hn.data(), dn.p, sizeof(double) * 2 * ncol, hipMemcpyDeviceToHost,
+                             st));
+      SU2_HIP(hipStreamSynchronize(st));
+      converged = true;
+      worst = 0;
+      bool left = false;
+      for (int b = 0; b < nb; ++b) {
+        if (!active[b]) continue;
+        double v;
+        std::memcpy(&v, &hoff[b], sizeof v);
+        if (v >= 2.0) {   // some pair still rotated this sweep
+          converged = false;
+          worst = std::max(worst, v - 2.0);
+        } else {
+          active[b] = 0;
+          left = true;
+        }
+      }
+      // columns that fell to the rounding level leave the schedule too
+      const bool shrunk = count_kept();
+      if ((left || shrunk) && !converged) {
+        build_schedule();
+        upload_jobs();
       }
     }
-    SU2_HIP(hipGetLastError());
-    SU2_HIP(hipMemcpyAsync(hoff.data(), doff.p, sizeof(unsigned long long) * nb,
-                           hipMemcpyDeviceToHost, st));
-    // the column norms for the next sweep's order (or the final one) come
-    // back with the counters: one wait per sweep
-    hipLaunchKernelGGL(colnorm_batched_kernel, dim3((unsigned)ncol), dim3(256), 0, st,
-                       (const BlockDesc*)ddesc.p, (const long long*)dnoff.p, nb, (long long)ncol,
-                       (double*)dn.p);
-    SU2_HIP(hipMemcpyAsync(hn.data(), dn.p, sizeof(double) * 2 * ncol, hipMemcpyDeviceToHost,
-                           st));
-    SU2_HIP(hipStreamSynchronize(st));
-    converged = true;
-    worst = 0;
-    bool left = false;
+  } else {
+    // The kept columns' pairs of column blocks that still need a rotation: at
+    // the start of a sweep one Gram matrix of each block's kept columns says
+    // which, and only those are scheduled, packed into as few rounds as their
+    // blocks allow.  (The last sweeps rotate a few pairs among many.)  A block
+    // without any has converged.  The schedule follows from the block alone.
+    std::vector<std::unique_ptr<DevMem>> gram(nb);
+    for (int b = 0; b < nb; ++b)
+      gram[b].reset(new DevMem(c, sizeof(double) * (size_t)K[b] * K[b]));
+    auto build_schedule = [&]() {
+      rounds.clear();
+      all.clear();
+      std::vector<FlagJob> fj;
+      std::vector<size_t> f0(nb, 0);
+      GemmBatch g;
+      for (int b = 0; b < nb; ++b) {
+        if (!active[b]) continue;
+        const int kb = kept[b], ncb = (kb + CB - 1) / CB;
+        double* G = (double*)gram[b]->p;
+        f0[b] = fj.size();
+        if (kb < 2) continue;
+        g.add(G, kb, kb, kb, Wc[b], L[b], 1, Wc[b], L[b], 0, L[b]);
+        for (int i = 0; i < ncb; ++i)
+          for (int j = i; j < ncb; ++j) fj.push_back(FlagJob{G, kb, kb, i, j, desc[b].normF});
+      }
+      g.run(c);
+      std::vector<double> flag(fj.size());
+      if (!fj.empty()) {
+        DevMem df(c, sizeof(FlagJob) * fj.size()), dflag(c, sizeof(double) * fj.size());
+        SU2_HIP(hipMemcpyAsync(df.p, fj.data(), sizeof(FlagJob) * fj.size(), hipMemcpyHostToDevice,
+                               st));
+        hipLaunchKernelGGL(pair_flags_kernel, dim3((unsigned)fj.size()), dim3(256), 0, st,
+                           (const FlagJob*)df.p, CB, tol, kTolAbs, (double*)dflag.p);
+        SU2_HIP(hipGetLastError());
+        SU2_HIP(hipMemcpyAsync(flag.data(), dflag.p, sizeof(double) * fj.size(),
+                               hipMemcpyDeviceToHost, st));
+        SU2_HIP(hipStreamSynchronize(st));
+      }
+      worst = 0;
+      for (int b = 0; b < nb; ++b) {
+        if (!active[b]) continue;
+        const int kb = kept[b], ncb = (kb + CB - 1) / CB;
+        auto width = [&](int i) { return std::min(CB, kb - i * CB); };
+        // blocks whose own columns need rotations, and the pairs that do
+        std::vector<char> self(ncb, 0);
+        std::vector<std::pair<int, int>> pairs;
+        std::vector<char> need((size_t)ncb * ncb, 0);
+        if (kb >= 2) {
+          size_t f = f0[b];
+          for (int i = 0; i < ncb; ++i)
+            for (int j = i; j < ncb; ++j, ++f) {
+              worst = std::max(worst, flag[f]);
+              if (!(flag[f] > 0.0)) continue;
+              if (i == j) self[i] = 1;
+              else need[(size_t)i * ncb + j] = 1;
+            }
+        }
+        // round-robin order, which spreads a block's pairs over the rounds
+        const int mp = ncb + (ncb & 1);
+        for (int r = 0; r < mp - 1; ++r)
+          for (int k = 0; k < mp / 2; ++k) {
+            const int x = (k == 0) ? mp - 1 : (r + k) % (mp - 1);
+            const int y = (k == 0) ? r : (r - k + (mp - 1)) % (mp - 1);
+            const int i = std::min(x, y), j = std::max(x, y);
+            if (j < ncb && need[(size_t)i * ncb + j]) pairs.push_back({i, j});
+          }
+        std::vector<std::vector<char>> used;   // used[round][column block]
+        std::vector<char> seen(ncb, 0);
+        auto place = [&](int i, int j) {
+          size_t r = 0;
+          for (; r < used.size(); ++r)
+            if (!used[r][i] && !used[r][j]) break;
+          if (r == used.size()) used.push_back(std::vector<char>(ncb, 0));
+          used[r][i] = used[r][j] = 1;
+          if (rounds.size() <= r) rounds.resize(r + 1);
+          PairJob J{b, i * CB, width(i), 0, 0, 1, 0};
+          if (j != i) {
+            J.q0 = j * CB;
+            J.bq = width(j);
+          }
+          rounds[r].push_back(J);
+        };
+        for (auto& pr : pairs) {
+          place(pr.first, pr.second);
+          seen[pr.first] = seen[pr.second] = 1;
+        }
+        // blocks in no pair: two by two, or alone
+        int open = -1;
+        for (int i = 0; i < ncb; ++i) {
+          if (!self[i] || seen[i]) continue;
+          if (open < 0) {
+            open = i;
+            continue;
+          }
+          place(open, i);
+          seen[open] = seen[i] = 1;
+          open = -1;
+        }
+        if (open >= 0) place(open, open);
+        if (used.empty()) {
+          active[b] = 0;
+          continue;
+        }
+        // the first visit of a block whose own columns need rotations sweeps
+        // all columns of its pair
+        std::vector<char> done(ncb, 0);
+        for (size_t r = 0; r < used.size(); ++r)
+          for (PairJob& J : rounds[r]) {
+            if (J.blk != b) continue;
+            const int i = J.p0 / CB, j = J.bq ? J.q0 / CB : i;
+            J.full = J.bq == 0 || (self[i] && !done[i]) || (self[j] && !done[j]);
+            done[i] = done[j] = 1;
+          }
+      }
+      slice_rounds();
+    };
+    // buffers for the most pairs a round can hold: half the column blocks of
+    // every block (or one block alone)
+    size_t pair_cap = 0;
+    for (int b = 0; b < nb; ++b) pair_cap += std::max(1, ((K[b] + CB - 1) / CB + 1) / 2);
+    const size_t gsz = (size_t)(NP / 16) * (NP / 16 + 1) / 2 * 256;
+    DevMem dgpart(c, sizeof(double) * gsz * MAX_SLICES * pair_cap);
+    DevMem drot(c, sizeof(double) * 2 * NP * NP * pair_cap), dact(c, sizeof(int) * 2 * pair_cap);
+    int lmax = 0, kmax = 0;
     for (int b = 0; b < nb; ++b) {
-      if (!active[b]) continue;
-      double v;
-      std::memcpy(&v, &hoff[b], sizeof v);
-      if (v >= 2.0) {   // some pair still rotated this sweep
-        converged = false;
-        worst = std::max(worst, v - 2.0);
-      } else {
-        active[b] = 0;
-        left = true;
-      }
+      lmax = std::max(lmax, L[b]);
+      kmax = std::max(kmax, K[b]);
     }
-    // columns that fell to the rounding level leave the schedule too
-    const bool shrunk = count_kept();
-    if ((left || shrunk) && !converged) {
+    const int rows_per_tile = (CB == 32 ? SolveThreads<32>::value : SolveThreads<16>::value) / 4;
+    const int wt = (lmax + rows_per_tile - 1) / rows_per_tile;
+    const int vt = (kmax + rows_per_tile - 1) / rows_per_tile;
+    // one round's three launches; round -1 of the next call: only V's rotations
+    auto run_rounds = [&](auto cb) {
+      constexpr int B = decltype(cb)::value;
+      constexpr int NT = SolveThreads<B>::value;
+      const BlockDesc* dd = (const BlockDesc*)ddesc.p;
+      DevMem djobs(c, sizeof(PairJob) * all.size());
+      SU2_HIP(hipMemcpyAsync(djobs.p, all.data(), sizeof(PairJob) * all.size(),
+                             hipMemcpyHostToDevice, st));
+      const PairJob* prev = nullptr;
+      int nprev = 0;
+      const double* prot = nullptr;
+      const int* pact = nullptr;
+      for (size_t r = 0; r <= rounds.size(); ++r) {
+        const bool tail = r == rounds.size();
+        const int nj = tail ? 0 : round_off[r + 1] - round_off[r];
+        const int pm = tail ? 1 : round_pmax[r];
+        const PairJob* jr = (const PairJob*)djobs.p + (tail ? 0 : round_off[r]);
+        double* rot = (double*)drot.p + (r & 1) * (size_t)NP * NP * pair_cap;
+        int* act = (int*)dact.p + (r & 1) * pair_cap;
+        SU2_CHECK((size_t)nj <= pair_cap, kErrCapacity, "jacobi: %d pairs in a round", nj);
+        if (nj > 0)
+          hipLaunchKernelGGL(gram_kernel<B>, dim3(nj * pm), dim3(256), 0, st, dd, jr, pm,
+                             (double*)dgpart.p);
+        if (nj + nprev > 0)
+          hipLaunchKernelGGL(solve_kernel<B>, dim3(nj + nprev * vt), dim3(NT), 0, st, dd, jr, nj,
+                             pm, (const double*)dgpart.p, tol, kTolAbs, inner_sweeps, rot, act,
+                             prev, vt, prot, pact);
+        if (nj > 0)
+          hipLaunchKernelGGL(apply_kernel<B>, dim3(nj * wt), dim3(NT), 0, st, dd, jr, wt,
+                             (const double*)rot, (const int*)act);
+        prev = jr;
+        nprev = nj;
+        prot = rot;
+        pact = act;
+      }
+      SU2_HIP(hipGetLastError());
+    };
+    for (int sweep = 0; sweep <= max_sweeps; ++sweep) {
+      // descending column norms (hn: read back after the previous sweep)
+      sort_permute();
+      count_kept();
       build_schedule();
-      SU2_CHECK(gpart_max <= gpart_cap, kErrCapacity, "jacobi: %zu partial Gram matrices",
-                gpart_max);
-      upload_jobs();
+      converged = all.empty();
+      if (converged || sweep == max_sweeps) break;
+      ++sweeps_done;
+      if (CB == 16) run_rounds(std::integral_constant<int, 16>{});
+      else run_rounds(std::integral_constant<int, 32>{});
+      norms();
     }
   }
   // Out of sweeps: the columns are accepted when orthogonal to 1e-6 of their
@@ -1119,15 +1826,15 @@ static int jacobi_svd_large(Context& c, const std::vector<JacobiBlock*>& blocks,
 
 int jacobi_svd_batched(Context& c, std::vector<JacobiBlock>& blocks, double tol, int max_sweeps,
                        int block_cols, int inner_sweeps, double* worst_out,
-                       int precondition_min_k) {
+                       int precondition_min_k, bool plain) {
   // a block's own shape decides, so its bits do not depend on the rest of
   // the batch
   std::vector<JacobiBlock*> small, large;
-  for (JacobiBlock& b : blocks) (small_svd_fits(b.m, b.n) ? small : large).push_back(&b);
+  for (JacobiBlock& b : blocks) (!plain && small_svd_fits(b.m, b.n) ? small : large).push_back(&b);
   double w1 = 0.0, w2 = 0.0;
   const int n1 = small_svd_batched(c, small, tol, kTolAbs, kNoiseRel, max_sweeps, &w1);
   const int n2 = jacobi_svd_large(c, large, tol, max_sweeps, block_cols, inner_sweeps, &w2,
-                                  precondition_min_k);
+                                  precondition_min_k, plain);
   if (worst_out) *worst_out = std::max(w1, w2);
   return std::max(n1, n2);
 }

@@ -12,21 +12,33 @@
 //
 // Blocks that fit one CU's LDS are decomposed there by one workgroup each
 // (small_svd.hpp); the rest of this description is about the larger ones.
-// Columns are cut into blocks of 16 (or 32).  A sweep visits every pair of blocks
-// once, in round-robin rounds of disjoint pairs; two kernel launches run all
-// pairs of a round for every block of the batch.  The first forms partial
-// Gram matrices (up to 64 x 64) of each pair over row slices of W, the second
-// sums them, diagonalises the pair's Gram matrix in LDS by parallel cyclic
-// Jacobi (one to three inner sweeps per visit) and applies the eigenvector
-// matrix to the pair's columns of W and V, each slice to its own rows.  A
-// round with few pairs cuts every pair into up to 8 slices so that it spans
-// the chip.  Before each sweep the columns are put in descending norm order.
+// Columns are cut into blocks of 16 (or 32), and before each sweep they are put
+// in descending norm order.  Two iterations rotate them:
+//
+// The usual one starts from QR-preconditioned columns (precond.hpp: every
+// block under 256 columns, and from the caller's limit on; what the first
+// pass leaves below 3e-8 of the block a second time).  A sweep begins with the
+// Gram matrix of the columns above the rounding level, which says which pairs
+// of column blocks still need a rotation; only those are visited, in rounds
+// of disjoint pairs, with three launches per round: partial Gram matrices of
+// the pairs over row slices of W, one workgroup per pair that diagonalises
+// its (up to 64 x 64) Gram matrix in LDS by parallel cyclic Jacobi, p columns
+// against q columns (all of them in a block's first visit), and the pairs'
+// columns of W times the result (V's a round later, beside the next
+// diagonalisations).  A block is done when no pair needs a rotation.
+//
+// The plain one visits every pair once per sweep with two launches per round
+// (Gram matrices, then every row slice diagonalises the whole pair for itself
+// and rotates its rows of W and V), preconditioned from the caller's limit on
+// only.  It is kept for uncut SVD calls (svd.hpp says why).  Measured against
+// it: svd call of a d = 500 step 20.7 -> 9.6 ms, d = 2000 83 -> 47 ms; 192 x
+// 192 block 14.1 -> 5.2 ms.
+//
 // Sweeps stop when every pair is orthogonal to
 // |g_ij| <= max(tol * sqrt(g_ii g_jj), 1e-14 ||A||_F (sqrt g_ii + sqrt g_jj))
 // (the absolute floor ends the iteration on columns that carry rounding
 // errors of order eps ||A||); columns with norm <= 1e-13 ||A||_F are left
-// out of the test.  A block that fits one column block is one self-pair per
-// sweep.
+// out of the test.
 #pragma once
 
 #include <vector>
@@ -58,9 +70,11 @@ struct JacobiBlock {
 // the call throws).
 // precondition_min_k: QR-precondition the blocks with precondition_min_k <=
 // min(m, n) <= kPrecondMaxK first (precond.hpp; 0: none); the results differ
-// from the plain iteration's by rounding only.
+// from the unpreconditioned iteration's by rounding only.
+// plain: the plain iteration, for every block.
 int jacobi_svd_batched(Context& c, std::vector<JacobiBlock>& blocks, double tol = 1e-13,
                        int max_sweeps = 60, int block_cols = 32, int inner_sweeps = 1,
-                       double* worst_out = nullptr, int precondition_min_k = 0);
+                       double* worst_out = nullptr, int precondition_min_k = 0,
+                       bool plain = false);
 
 }  // namespace su2

@@ -165,10 +165,14 @@ std::vector<SvdResult> truncated_svd_batch(Context& c, const std::vector<SvdJob>
   int jacobi_sweeps = 0;
   double t_jacobi = 0, jacobi_worst = 0;
   {
-    std::vector<JacobiBlock> jb;
-    std::vector<std::pair<size_t, size_t>> idx;
+    // by the iteration asked for: [0] the usual one, [1] the plain one
+    std::vector<JacobiBlock> jb[2];
+    std::vector<std::pair<size_t, size_t>> idx[2];
     for (size_t q = 0; q < jobs.size(); ++q) {
       wv[q].resize(secs[q].size());
+      long long columns = 0;
+      for (const Sec& s : secs[q]) columns += s.k;
+      const int plain = jobs[q].keep_all_plain && jobs[q].max_dcut >= columns;
       for (size_t i = 0; i < secs[q].size(); ++i) {
         Sec& s = secs[q][i];
         if (s.k == 0) continue;
@@ -182,19 +186,27 @@ std::vector<SvdResult> truncated_svd_batch(Context& c, const std::vector<SvdJob>
         b.W = s.U.p;
         b.V = s.V.p;
         b.group = (int)q;
-        jb.push_back(b);
-        idx.push_back({q, i});
+        jb[plain].push_back(b);
+        idx[plain].push_back({q, i});
       }
     }
     const auto tj = std::chrono::steady_clock::now();
-    jacobi_sweeps = jacobi_svd_batched(c, jb, 1e-13, 60, c.svd_block_cols, c.svd_inner_sweeps,
-                                       &jacobi_worst, c.svd_precondition_min_k);
-    t_jacobi = std::chrono::duration<double>(std::chrono::steady_clock::now() - tj).count();
-    for (size_t t = 0; t < jb.size(); ++t) {
-      std::vector<double>& w = wv[idx[t].first][idx[t].second];
-      w.resize(jb[t].s.size());
-      for (size_t q = 0; q < w.size(); ++q) w[q] = jb[t].s[q] * jb[t].s[q];
+    for (int plain = 0; plain < 2; ++plain) {
+      double w = 0;
+      jacobi_sweeps = std::max(
+          jacobi_sweeps, jacobi_svd_batched(c, jb[plain], 1e-13, 60, c.svd_block_cols,
+                                            c.svd_inner_sweeps, &w, c.svd_precondition_min_k,
+                                            plain != 0));
+      jacobi_worst = std::max(jacobi_worst, w);
     }
+    t_jacobi = std::chrono::duration<double>(std::chrono::steady_clock::now() - tj).count();
+    for (int plain = 0; plain < 2; ++plain)
+      for (size_t t = 0; t < jb[plain].size(); ++t) {
+        std::vector<double>& w = wv[idx[plain][t].first][idx[plain][t].second];
+        const std::vector<double>& sv = jb[plain][t].s;
+        w.resize(sv.size());
+        for (size_t q = 0; q < w.size(); ++q) w[q] = sv[q] * sv[q];
+      }
   }
   // column factors of every sector of every wavefunction: one upload, the
   // scalings queued, no wait until the outputs are in place
@@ -225,8 +237,9 @@ std::vector<SvdResult> truncated_svd_batch(Context& c, const std::vector<SvdJob>
   return out;
 }
 
-SvdResult truncated_svd(Context& c, const Tensor& psi, double p1, double p2, int max_dcut) {
-  std::vector<SvdJob> jobs{SvdJob{&psi, p1, p2, max_dcut}};
+SvdResult truncated_svd(Context& c, const Tensor& psi, double p1, double p2, int max_dcut,
+                        bool keep_all_plain) {
+  std::vector<SvdJob> jobs{SvdJob{&psi, p1, p2, max_dcut, keep_all_plain}};
   std::vector<SvdResult> r = truncated_svd_batch(c, jobs);
   return std::move(r[0]);
 }
