@@ -60,17 +60,15 @@ HeffBatch::Pattern& HeffBatch::pattern(const std::vector<Req>& reqs) {
   if (it != cache_.end()) return *it->second;
   std::unique_ptr<Pattern> P(new Pattern());
   P->nreq = (int)reqs.size();
-  int var[2][2] = {{-1, -1}, {-1, -1}};   // [prec][stage]: the first plan's variants
+  int var[2][2] = {{-1, -1}, {-1, -1}};   // [prec][stage]: the first pinned variants
   for (auto& r : reqs) {
     HeffPlan& h = *r.plan;
     const int pi = (int)r.prec;
     if (r.prec == Prec::F32) h.ensure_fp32();
     GroupedGemm& g1 = r.prec == Prec::F64 ? h.stage1_ : *h.stage1_32_;
     GroupedGemm& g2 = r.prec == Prec::F64 ? h.stage2_ : *h.stage2_32_;
-    if (var[pi][0] < 0) {
-      var[pi][0] = g1.variant();
-      var[pi][1] = g2.variant();
-    }
+    if (var[pi][0] < 0) var[pi][0] = g1.pinned_variant();
+    if (var[pi][1] < 0) var[pi][1] = g2.pinned_variant();
     P->s1[pi].append(g1);
     P->s2[pi].append(g2);
     P->max_in = std::max(P->max_in, h.psi_size_);

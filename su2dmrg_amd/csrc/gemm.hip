@@ -729,6 +729,25 @@ const VariantInfo& variant_info(Prec p, int v) {
   return p == Prec::F64 ? kVariants64[v] : kVariants32[v];
 }
 int num_variants(Prec p) { return p == Prec::F64 ? kNumVariants64 : kNumVariants32; }
+// Variant of a launch that nobody pinned.  64 x 64 tiles are faster up to
+// about 6e10 flops a launch: with the sector dimensions in the hundreds a 128
+// x 128 grid leaves the chip partly idle and pads its edge tiles.  Past that
+// the 128 x 128 tiles' fewer operand reads count.  Measured on H_eff stages 1
+// and 2 (us, 128 x 128 against 64 x 64): centre bond d = 32 10 / 37 against 6
+// / 17; d = 500 92 / 110 against 75 / 92; d = 1000 558 / 705 against 524 /
+// 574; d = 2000 3496 / 3725 against 3696 / 4064; FP32 at d = 1000 321 / 377
+// against 320 / 319, at d = 2000 1886 / 1997 against 2157 / 2097.
+int default_variant(Prec p, double flops) {
+  if (flops < 6e10) return 4;
+  return p == Prec::F64 ? 1 : 0;
+}
+
+// Fewest k-tiles of a split.  Shorter splits put more workgroups on the
+// smallest launches but add partial sums to write and reduce: with 3 to 6 an
+// apply at d = 32 takes 20 to 22 us instead of 26, at d = 300 78 to 89 instead
+// of 72, and the 1000-wide one-term bond 150 to 178 instead of 118.
+constexpr int kMinKtPerSplit = 8;
+
 size_t elem_size(Prec p) { return p == Prec::F64 ? sizeof(double) : sizeof(float); }
 
 }  // namespace
@@ -817,11 +836,17 @@ void GroupedGemm::finalize(Context& c, int min_units, int kt_per_unit, int varia
   min_units_ = std::max(1, min_units);
   kt_per_unit_ = std::max(1, kt_per_unit);
   stream_ = c.stream();
-  set_variant(variant < 0 ? kDefaultGemmVariant : variant);
+  if (variant < 0) build(default_variant(prec_, flops_));
+  else set_variant(variant);
 }
 
 void GroupedGemm::set_variant(int v) {
   SU2_CHECK(v >= 0 && v < num_variants(prec_), kErrArgument, "gemm variant %d out of range", v);
+  pinned_ = true;
+  build(v);
+}
+
+void GroupedGemm::build(int v) {
   const VariantInfo& V = variant_info(prec_, v);
   release();
   variant_ = v;
@@ -850,11 +875,12 @@ void GroupedGemm::set_variant(int v) {
     // streams from HBM about once while the smaller one is re-read from cache
     p.n_fast = p.M > p.N ? 1 : 0;
     // K split from this problem's own shape only (see finalize)
-    const long long tiles = std::max(1LL, (long long)p.tiles_m * p.tiles_n);
+    const long long tiles =
+        std::max(1LL, (long long)((p.M + 63) / 64) * ((p.N + 63) / 64));
     const long long by_units = (min_units_ + tiles - 1) / tiles;
     const long long by_depth = p.kt_total / kt_per_unit_;
     const long long ks = std::max(by_units, by_depth);
-    p.ksplit = (int)std::max(1LL, std::min(ks, std::max(1LL, (long long)p.kt_total / 8)));
+    p.ksplit = (int)std::max(1LL, std::min(ks, std::max(1LL, (long long)p.kt_total / kMinKtPerSplit)));
   }
   // units in order of decreasing cost (stable), so that the cheap units of a
   // launch come last in the XCD ranges and fill their tails

@@ -61,10 +61,8 @@ struct ReduceProblem {
   long long elem_begin;
 };
 
-// Number of compiled tile variants (BM x BN x BK x waves) of a precision and
-// the default (the same index for both).
+// Number of compiled tile variants (BM x BN x BK x waves) of a precision.
 int gemm_num_variants(Prec p = Prec::F64);
-constexpr int kDefaultGemmVariant = 1;
 
 // Host-side plan: build problems, then finalize once; launch many times.
 class GroupedGemm {
@@ -85,16 +83,20 @@ class GroupedGemm {
   void append(const GroupedGemm& other);
   Prec prec() const { return prec_; }
   // Chooses the K split of every problem and uploads the tables for tile
-  // variant `variant` (-1: default), in device memory of `c` (the plan then
-  // launches on any stream but must not outlive c).  A problem's split
-  // follows from the problem alone, so its summation order, and its bits, do
-  // not depend on what else shares the launch: enough splits for about
-  // min_units work units of its own, or one split per kt_per_unit k-tiles,
-  // whichever is more, with at least 8 k-tiles per split.
+  // variant `variant` (-1: the launch's own choice, default_variant in
+  // gemm.hip), in device memory of `c` (the plan then launches on any stream
+  // but must not outlive c).  A problem's split follows from the problem
+  // alone, and not from the tile either, so its summation order, and its bits,
+  // do not depend on what else shares the launch: enough splits for about
+  // min_units 64 x 64 tiles' worth of units of its own, or one split per
+  // kt_per_unit k-tiles, whichever is more, with at least kMinKtPerSplit
+  // k-tiles per split.
   void finalize(Context& c, int min_units, int kt_per_unit, int variant = -1);
-  // Re-tiles for another variant (device tables rebuilt).
+  // Re-tiles for another variant (device tables rebuilt) and keeps it.
   void set_variant(int v);
   int variant() const { return variant_; }
+  // the variant that set_variant (or autotune) asked for, -1 if none did
+  int pinned_variant() const { return pinned_ ? variant_ : -1; }
   // Launches whose slices share one layout (op(B) = B, op(A) fixed) run the
   // straight-line uniform kernel unless this is switched off (before
   // finalize or set_variant); layout() is 0 (NN), 1 (TN) or -1 (mixed).
@@ -112,6 +114,7 @@ class GroupedGemm {
 
  private:
   void release();
+  void build(int v);
   std::vector<GemmProblem> probs_;      // as added
   std::vector<GemmSlice> slices_;
   std::vector<GemmProblem> run_probs_;  // tiled for the current variant
@@ -130,6 +133,7 @@ class GroupedGemm {
   std::shared_ptr<DevicePool> pool_;   // device memory of the finalizing context
   hipStream_t stream_ = nullptr;       // the finalizing context's stream (table uploads)
   int variant_ = -1;
+  bool pinned_ = false;
   int layout_ = -1;
   bool uniform_ = true;
   Prec prec_ = Prec::F64;
