@@ -69,15 +69,6 @@ __global__ void move_batch_kernel(const VecMove* __restrict__ desc) {
   }
 }
 
-// x *= 1 / sqrt(s[0]) with s read on the device (normalisation without a
-// host round trip)
-__global__ void scal_inv_sqrt_kernel(double* x, long long n, const double* __restrict__ s) {
-  const double a = 1.0 / sqrt(s[0]);
-  long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  long long stride = (long long)gridDim.x * blockDim.x;
-  for (; i < n; i += stride) x[i] *= a;
-}
-
 __global__ void copy_kernel(double* __restrict__ y, const double* __restrict__ x, long long n) {
   long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   long long stride = (long long)gridDim.x * blockDim.x;
@@ -351,13 +342,6 @@ void dev_move_batch(Context& c, const VecMove* d_desc, int ndesc, long long max_
   unsigned gx = grid_for(max_n);
   if (gx > 1024) gx = 1024;
   hipLaunchKernelGGL(move_batch_kernel, dim3(gx, ndesc), dim3(kThreads), 0, c.stream(), d_desc);
-  SU2_HIP(hipGetLastError());
-}
-
-void dev_scal_inv_sqrt(Context& c, double* x, long long n, const double* d_s) {
-  if (n <= 0) return;
-  hipLaunchKernelGGL(scal_inv_sqrt_kernel, dim3(grid_for(n)), dim3(kThreads), 0, c.stream(), x, n,
-                     d_s);
   SU2_HIP(hipGetLastError());
 }
 

@@ -29,8 +29,6 @@ struct VecMove {
   int mode, pad;
 };
 void dev_move_batch(Context& c, const VecMove* d_desc, int ndesc, long long max_n);
-// x *= 1 / sqrt(s[0]), s in device memory (no wait)
-void dev_scal_inv_sqrt(Context& c, double* x, long long n, const double* d_s);
 // FP32 buffers of the mixed-precision matvec: fill, round to FP32, widen
 void dev_fill_f32(Context& c, float* x, long long n, float v);
 void dev_convert_f64_f32(Context& c, float* y, const double* x, long long n);

@@ -4,9 +4,9 @@
 #include <cmath>
 #include <numeric>
 
-#include "blas1.hpp"
 #include "common.hpp"
 #include "context.hpp"
+#include "krylov.hpp"
 
 namespace su2 {
 
@@ -92,14 +92,16 @@ struct LzJob {
   LanczosJob* job;
   int st = kStart;
   int m = 0;
-  std::vector<DevBuf> ff;   // Krylov vectors 0..mlanc
+  DevBuf ff;                // Krylov vectors 0..mlanc, ld apart
+  long long ld = 0;
   DevBuf tmp;
-  std::vector<double> aal, nnl, z;
-  int slot0 = 0;            // first of this job's slots in the shared scalar array
+  std::vector<double> aal, nnl;
+  double* slots = nullptr;  // alpha, a, b (pinned)
   bool pending = false;     // has a matvec request this round
   const double* x = nullptr;
   double* y = nullptr;
   bool check = false;
+  double* v(int k) const { return ff.p + k * ld; }
 };
 
 }  // namespace
@@ -107,35 +109,24 @@ struct LzJob {
 void lanczos_batch(Context& c, std::vector<LanczosJob>& jobs, const BatchApply& apply) {
   const int nj = (int)jobs.size();
   if (nj == 0) return;
-  // device scalars of every job: coef[0..mlanc] (alphas and the current
-  // reorthogonalisation coefficient), then A and B (norms, overlaps)
-  int per = 0;
-  for (auto& j : jobs) {
-    SU2_CHECK(j.mlanc >= 2, kErrArgument, "lanczos: mlanc=%d", j.mlanc);
-    per = std::max(per, j.mlanc + 3);
-  }
-  DevBuf scal(c, (long long)per * nj);
-  std::vector<double> host((size_t)per * nj, 0.0);
-  dev_fill(c, scal.p, (long long)per * nj, 0.0);
+  // alpha, a and b of every job, written by the device into pinned memory (the
+  // applies below leave the context's host scratch alone)
+  double* host = c.host_scratch(3 * (size_t)nj);
+  DevBuf part(c, krylov_partials(nj));
   std::vector<LzJob> L(nj);
   for (int i = 0; i < nj; ++i) {
     LzJob& s = L[i];
     s.job = &jobs[i];
+    SU2_CHECK(s.job->mlanc >= 2, kErrArgument, "lanczos: mlanc=%d", s.job->mlanc);
     s.job->res = LanczosResult();
     const long long n = std::max<long long>(s.job->n, 1);
-    s.ff.reserve(s.job->mlanc + 1);
-    for (int k = 0; k <= s.job->mlanc; ++k) s.ff.emplace_back(c, n);
+    s.ld = (n + 31) / 32 * 32;
+    s.ff = DevBuf(c, s.ld * (s.job->mlanc + 1));
     s.tmp = DevBuf(c, n);
     s.aal.assign(s.job->mlanc, 0.0);
     s.nnl.assign(s.job->mlanc + 1, 0.0);
-    s.slot0 = i * per;
+    s.slots = host + 3 * i;
   }
-  auto coef = [&](LzJob& s, int k) { return scal.p + s.slot0 + k; };
-  auto A = [&](LzJob& s) { return scal.p + s.slot0 + s.job->mlanc + 1; };
-  auto B = [&](LzJob& s) { return scal.p + s.slot0 + s.job->mlanc + 2; };
-  auto hcoef = [&](LzJob& s, int k) { return host[s.slot0 + k]; };
-  auto hA = [&](LzJob& s) { return host[s.slot0 + s.job->mlanc + 1]; };
-  auto hB = [&](LzJob& s) { return host[s.slot0 + s.job->mlanc + 2]; };
   auto request = [&](LzJob& s, const double* x, double* y, bool check) {
     s.pending = true;
     s.x = x;
@@ -145,21 +136,18 @@ void lanczos_batch(Context& c, std::vector<LanczosJob>& jobs, const BatchApply& 
     if (check && s.job->mixed) ++s.job->res.check_matvecs;
   };
   // Ritz vector of the m x m tridiagonal into psi, then psi normalised on
-  // the device (the check's normalisation, lanczos_su2.cpp:320-332)
+  // the device (the check's normalisation, lanczos_su2.cpp:320-332); the
+  // jobs of a round are queued together
+  std::vector<KrylovRitz> ritzes;
   auto ritz = [&](LzJob& s, int m, bool normalise) {
-    const long long n = s.job->n;
     std::vector<double> d(s.aal.begin(), s.aal.begin() + m), e(s.nnl.begin() + 1, s.nnl.begin() + m),
         w, z;
     tridiag_eig(d, e, w, z);
+    z.resize(m);
     if (z[0] < 0)   // Ritz vector with a positive overlap on the start vector
       for (int j = 0; j < m; ++j) z[j] = -z[j];
-    dev_fill(c, s.job->psi, n, 0.0);
-    for (int j = 0; j < m; ++j) dev_axpy(c, s.job->psi, s.ff[j].p, n, z[j]);
+    ritzes.push_back(KrylovRitz{s.ff.p, s.ld, s.job->n, s.job->psi, z, normalise, s.slots + 1});
     s.job->res.ritz = s.job->res.energy = w[0];
-    if (normalise) {
-      dev_dot_to(c, s.job->psi, s.job->psi, n, A(s));
-      dev_scal_inv_sqrt(c, s.job->psi, n, A(s));
-    }
   };
   auto check_request = [&](LzJob& s, int st) {
     ritz(s, s.m, true);
@@ -169,24 +157,22 @@ void lanczos_batch(Context& c, std::vector<LanczosJob>& jobs, const BatchApply& 
   // after iteration m: the next Krylov matvec, or the last one
   auto advance = [&](LzJob& s) {
     ++s.m;
-    if (s.m < s.job->mlanc) {
-      request(s, s.ff[s.m - 1].p, s.ff[s.m].p, false);
-      s.st = kLoop;
-    } else {
-      request(s, s.ff[s.job->mlanc - 1].p, s.ff[s.job->mlanc].p, false);
-      s.st = kFinal;
-    }
+    request(s, s.v(s.m - 1), s.v(s.m), false);
+    s.st = s.m < s.job->mlanc ? kLoop : kFinal;
+  };
+  std::vector<KrylovOp> ops;
+  auto queue = [&](LzJob& s, int kind, int m, double beta) {
+    ops.push_back(KrylovOp{kind, m, s.ff.p, s.ld, s.job->n, s.job->psi, s.tmp.p, beta, s.slots,
+                           s.slots + 1, s.slots + 2});
   };
 
-  // start: ff[0] = psi / |psi| (initialize_lanczos, lanczos_su2.cpp:36-47)
+  // start: v[0] = psi / |psi| (initialize_lanczos, lanczos_su2.cpp:36-47)
   for (auto& s : L) {
-    const long long n = s.job->n;
-    dev_dot_to(c, s.job->psi, s.job->psi, n, B(s));
-    dev_copy(c, s.ff[0].p, s.job->psi, n);
-    dev_scal_inv_sqrt(c, s.ff[0].p, n, B(s));
-    request(s, s.ff[0].p, s.ff[1].p, false);
+    queue(s, kKrylovNormalise, 0, 0.0);
+    request(s, s.v(0), s.v(1), false);
     s.st = kAfterFirst;
   }
+  krylov_run(c, ops, part.p);
   bool first = true;
   for (;;) {
     std::vector<LanczosReq> reqs;
@@ -195,84 +181,58 @@ void lanczos_batch(Context& c, std::vector<LanczosJob>& jobs, const BatchApply& 
     if (reqs.empty()) break;
     apply(reqs);
     // each job's vector algebra after its matvec, scalars into its slots
+    ops.clear();
     for (auto& s : L) {
       if (!s.pending) continue;
       s.pending = false;
-      const long long n = s.job->n;
-      const int m = s.m;
       switch (s.st) {
-        case kAfterFirst:
-          dev_dot_to(c, s.ff[0].p, s.ff[1].p, n, coef(s, 0));
-          dev_axpy_dev(c, s.ff[1].p, s.ff[0].p, n, coef(s, 0), -1.0);
-          dev_dot_to(c, s.ff[1].p, s.ff[1].p, n, A(s));
-          break;
-        case kM2Final:
-          dev_dot_to(c, s.ff[1].p, s.ff[2].p, n, coef(s, 1));
-          break;
-        case kLoop:
-          dev_dot_to(c, s.ff[m - 1].p, s.ff[m].p, n, coef(s, m - 1));
-          dev_axpy_dev(c, s.ff[m].p, s.ff[m - 1].p, n, coef(s, m - 1), -1.0);
-          dev_axpy(c, s.ff[m].p, s.ff[m - 2].p, n, -s.nnl[m - 1]);
-          for (int j = 0; j < m; ++j) {
-            dev_dot_to(c, s.ff[m].p, s.ff[j].p, n, coef(s, s.job->mlanc));
-            dev_axpy_dev(c, s.ff[m].p, s.ff[j].p, n, coef(s, s.job->mlanc), -1.0);
-          }
-          dev_dot_to(c, s.ff[m].p, s.ff[m].p, n, A(s));
-          break;
+        case kAfterFirst: queue(s, kKrylovFirst, 1, 0.0); break;
+        case kM2Final: queue(s, kKrylovOverlap, 2, 0.0); break;
+        case kLoop: queue(s, kKrylovStep, s.m, s.nnl[s.m - 1]); break;
         case kCheckCont:
-        case kCheckDone:
-          dev_dot_to(c, s.tmp.p, s.tmp.p, n, A(s));
-          dev_dot_to(c, s.tmp.p, s.job->psi, n, B(s));
-          break;
-        case kFinal:
-          dev_dot_to(c, s.ff[s.job->mlanc - 1].p, s.ff[s.job->mlanc].p, n,
-                     coef(s, s.job->mlanc - 1));
-          break;
-        default:
-          break;
+        case kCheckDone: queue(s, kKrylovCheck, 0, 0.0); break;
+        case kFinal: queue(s, kKrylovOverlap, s.job->mlanc, 0.0); break;
+        default: break;
       }
     }
+    krylov_run(c, ops, part.p);
     // one wait for the scalars of every job
-    SU2_HIP(hipMemcpyAsync(host.data(), scal.p, sizeof(double) * host.size(),
-                           hipMemcpyDeviceToHost, c.stream()));
     SU2_HIP(hipStreamSynchronize(c.stream()));
     for (auto& s : L) {
       if (s.st == kDone || s.pending) continue;
-      const long long n = s.job->n;
       const int mlanc = s.job->mlanc;
+      const double alpha = s.slots[0], a = s.slots[1], b = s.slots[2];
       switch (s.st) {
         case kAfterFirst: {
-          if (first) SU2_CHECK(hB(s) > 0, kErrNumeric, "lanczos: zero start vector");
-          s.aal[0] = hcoef(s, 0);
-          s.nnl[1] = std::sqrt(hA(s));
+          if (first) SU2_CHECK(b > 0, kErrNumeric, "lanczos: zero start vector");
+          s.aal[0] = alpha;
           // an exactly invariant start vector (a 1-dim H_eff) leaves nnl = 0:
           // the unnormalised residual is then never read again
-          if (s.nnl[1] > 0) dev_scal(c, s.ff[1].p, n, 1.0 / s.nnl[1]);
+          s.nnl[1] = std::sqrt(a);
           if (mlanc == 2) {
             if (s.nnl[1] < s.job->tol) {
               ritz(s, 1, false);
               s.st = kDone;
             } else {
-              request(s, s.ff[1].p, s.ff[2].p, false);
+              request(s, s.v(1), s.v(2), false);
               s.st = kM2Final;
             }
           } else {
             s.m = 2;
-            request(s, s.ff[1].p, s.ff[2].p, false);
+            request(s, s.v(1), s.v(2), false);
             s.st = kLoop;
           }
           break;
         }
         case kM2Final:
-          s.aal[1] = hcoef(s, 1);
+          s.aal[1] = alpha;
           ritz(s, 2, true);
           s.st = kDone;
           break;
         case kLoop: {
           const int m = s.m;
-          s.aal[m - 1] = hcoef(s, m - 1);
-          s.nnl[m] = std::sqrt(hA(s));
-          if (s.nnl[m] > 0) dev_scal(c, s.ff[m].p, n, 1.0 / s.nnl[m]);
+          s.aal[m - 1] = alpha;
+          s.nnl[m] = std::sqrt(a);
           if (s.nnl[m] < s.job->tol) check_request(s, kCheckDone);
           else if (m % 4 == 0) check_request(s, kCheckCont);
           else advance(s);
@@ -280,7 +240,7 @@ void lanczos_batch(Context& c, std::vector<LanczosJob>& jobs, const BatchApply& 
         }
         case kCheckCont:
         case kCheckDone: {
-          const double prod = std::sqrt(hA(s)), rq = hB(s);
+          const double prod = std::sqrt(a), rq = b;
           s.job->res.residual = std::sqrt(std::max(0.0, prod * prod - rq * rq));
           if (s.job->mixed) s.job->res.energy = rq;
           const double ov = std::fabs(rq / prod);
@@ -289,7 +249,7 @@ void lanczos_batch(Context& c, std::vector<LanczosJob>& jobs, const BatchApply& 
           break;
         }
         case kFinal:
-          s.aal[mlanc - 1] = hcoef(s, mlanc - 1);
+          s.aal[mlanc - 1] = alpha;
           s.m = mlanc;
           check_request(s, kCheckDone);
           break;
@@ -297,6 +257,8 @@ void lanczos_batch(Context& c, std::vector<LanczosJob>& jobs, const BatchApply& 
           break;
       }
     }
+    krylov_ritz(c, ritzes, part.p);
+    ritzes.clear();
     first = false;
   }
   SU2_HIP(hipStreamSynchronize(c.stream()));
