@@ -37,14 +37,8 @@ HeffBatch::~HeffBatch() { clear(); }
 void HeffBatch::release(Pattern& P) {
   if (P.exec) (void)hipGraphExecDestroy(P.exec);
   if (P.graph) (void)hipGraphDestroy(P.graph);
-  if (P.done) (void)hipEventDestroy(P.done);
-  if (P.h_desc) (void)hipHostFree(P.h_desc);
-  if (P.d_desc) c_.dev_free(P.d_desc);
   P.exec = nullptr;
   P.graph = nullptr;
-  P.done = nullptr;
-  P.h_desc = nullptr;
-  P.d_desc = nullptr;
 }
 
 void HeffBatch::clear() {
@@ -59,7 +53,6 @@ HeffBatch::Pattern& HeffBatch::pattern(const std::vector<Req>& reqs) {
   auto it = cache_.find(key);
   if (it != cache_.end()) return *it->second;
   std::unique_ptr<Pattern> P(new Pattern());
-  P->nreq = (int)reqs.size();
   int var[2][2] = {{-1, -1}, {-1, -1}};   // [prec][stage]: the first pinned variants
   for (auto& r : reqs) {
     HeffPlan& h = *r.plan;
@@ -67,56 +60,52 @@ HeffBatch::Pattern& HeffBatch::pattern(const std::vector<Req>& reqs) {
     if (r.prec == Prec::F32) h.ensure_fp32();
     GroupedGemm& g1 = r.prec == Prec::F64 ? h.stage1_ : *h.stage1_32_;
     GroupedGemm& g2 = r.prec == Prec::F64 ? h.stage2_ : *h.stage2_32_;
-    if (var[pi][0] < 0) var[pi][0] = g1.pinned_variant();
-    if (var[pi][1] < 0) var[pi][1] = g2.pinned_variant();
-    P->s1[pi].append(g1);
-    P->s2[pi].append(g2);
-    P->max_in = std::max(P->max_in, h.psi_size_);
+    if (reqs.size() == 1) {
+      // alone: the plan's own launches, no tables to build
+      P->run1.push_back(&g1);
+      P->run2.push_back(&g2);
+    } else {
+      if (var[pi][0] < 0) var[pi][0] = g1.pinned_variant();
+      if (var[pi][1] < 0) var[pi][1] = g2.pinned_variant();
+      P->s1[pi].append(g1);
+      P->s2[pi].append(g2);
+    }
     for (auto& z : h.zero_blocks_) {
       VecMove m{};
       m.dst = r.prec == Prec::F64 ? (void*)(h.d_out_ + z.first) : (void*)(h.d_out32_ + z.first);
       m.n = z.second;
       m.mode = r.prec == Prec::F64 ? kZeroF64 : kZeroF32;
       P->fill.push_back(m);
-      P->max_fill = std::max(P->max_fill, z.second);
     }
   }
-  P->max_out = P->max_in;
   for (int pi = 0; pi < 2; ++pi) {
-    if (P->s1[pi].nproblems() > 0) P->s1[pi].finalize(c_, kMinUnits1, kKtPerUnit1, var[pi][0]);
-    if (P->s2[pi].nproblems() > 0) P->s2[pi].finalize(c_, kMinUnits2, kKtPerUnit2, var[pi][1]);
+    if (P->s1[pi].nproblems() > 0) {
+      P->s1[pi].finalize(c_, kMinUnits1, kKtPerUnit1, var[pi][0]);
+      P->run1.push_back(&P->s1[pi]);
+    }
+    if (P->s2[pi].nproblems() > 0) {
+      P->s2[pi].finalize(c_, kMinUnits2, kKtPerUnit2, var[pi][1]);
+      P->run2.push_back(&P->s2[pi]);
+    }
   }
-  const size_t nd = 2 * reqs.size() + P->fill.size();
-  P->d_desc = (VecMove*)c_.dev_alloc(nd * sizeof(VecMove));
-  SU2_HIP(hipHostMalloc((void**)&P->h_desc, 2 * reqs.size() * sizeof(VecMove),
-                        hipHostMallocDefault));
-  if (!P->fill.empty())
-    SU2_HIP(hipMemcpyAsync(P->d_desc + 2 * reqs.size(), P->fill.data(),
-                           P->fill.size() * sizeof(VecMove), hipMemcpyHostToDevice, c_.stream()));
-  SU2_HIP(hipEventCreateWithFlags(&P->done, hipEventDisableTiming));
   Pattern& ref = *P;
   cache_[key] = std::move(P);
   return ref;
 }
 
-// inputs in, zero blocks, both stages of both precisions, outputs out
+// zero blocks and both stages of both precisions
 void HeffBatch::launch_body(Pattern& P) {
-  hipStream_t s = c_.stream();
-  dev_move_batch(c_, P.d_desc, P.nreq, P.max_in);
-  if (!P.fill.empty()) dev_move_batch(c_, P.d_desc + 2 * P.nreq, (int)P.fill.size(), P.max_fill);
-  for (int pi = 0; pi < 2; ++pi)
-    if (P.s1[pi].nproblems() > 0) P.s1[pi].launch(s);
-  for (int pi = 0; pi < 2; ++pi)
-    if (P.s2[pi].nproblems() > 0) P.s2[pi].launch(s);
-  dev_move_batch(c_, P.d_desc + P.nreq, P.nreq, P.max_out);
+  dev_moves(c_, P.fill);
+  for (const GroupedGemm* g : P.run1) g->launch(c_.stream());
+  for (const GroupedGemm* g : P.run2) g->launch(c_.stream());
 }
 
 void HeffBatch::apply(const std::vector<Req>& reqs) {
   if (reqs.empty()) return;
   c_.make_current();
   Pattern& P = pattern(reqs);
-  // the previous replay must have read the staged descriptors
-  if (P.used) SU2_HIP(hipEventSynchronize(P.done));
+  // every input and output of the round in one launch each
+  std::vector<VecMove> ins, outs;
   for (size_t i = 0; i < reqs.size(); ++i) {
     const Req& r = reqs[i];
     HeffPlan& h = *r.plan;
@@ -136,11 +125,10 @@ void HeffBatch::apply(const std::vector<Req>& reqs) {
       out.src = h.d_out32_;
       out.mode = kMoveF32toF64;
     }
-    P.h_desc[i] = in;
-    P.h_desc[reqs.size() + i] = out;
+    ins.push_back(in);
+    outs.push_back(out);
   }
-  SU2_HIP(hipMemcpyAsync(P.d_desc, P.h_desc, 2 * reqs.size() * sizeof(VecMove),
-                         hipMemcpyHostToDevice, c_.stream()));
+  dev_moves(c_, ins);
   if (!use_graph_) {
     launch_body(P);
   } else {
@@ -172,8 +160,7 @@ void HeffBatch::apply(const std::vector<Req>& reqs) {
     SU2_HIP(hipGraphLaunch(P.exec, c_.stream()));
     ++replays_;
   }
-  SU2_HIP(hipEventRecord(P.done, c_.stream()));
-  P.used = true;
+  dev_moves(c_, outs);
 }
 
 // ---------------------------------------------------------------------------

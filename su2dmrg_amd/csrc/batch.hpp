@@ -63,16 +63,12 @@ class HeffBatch {
 
  private:
   struct Pattern {
-    GroupedGemm s1[2], s2[2];   // by precision: F64, F32
+    GroupedGemm s1[2], s2[2];   // by precision: F64, F32 (several requests)
+    // what a launch runs: the above, or a single request's own plans
+    std::vector<const GroupedGemm*> run1, run2;
     std::vector<VecMove> fill;  // zero blocks of the outputs (fixed)
-    int nreq = 0;
-    long long max_in = 0, max_out = 0, max_fill = 0;
-    VecMove* d_desc = nullptr;  // [nreq in | nreq out | fill]
-    VecMove* h_desc = nullptr;  // pinned staging of the in/out descriptors
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
-    hipEvent_t done = nullptr;  // the last replay has read h_desc
-    bool used = false;
     Pattern() : s1{GroupedGemm(Prec::F64), GroupedGemm(Prec::F32)},
                 s2{GroupedGemm(Prec::F64), GroupedGemm(Prec::F32)} {}
   };

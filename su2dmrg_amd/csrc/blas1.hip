@@ -44,8 +44,13 @@ __global__ void f32_to_f64_kernel(double* __restrict__ y, const float* __restric
 // One launch for many vector moves: descriptor blockIdx.y, a grid-stride loop
 // over its elements (a copy, a rounding to FP32, a widening to FP64, or a
 // fill with zero).
-__global__ void move_batch_kernel(const VecMove* __restrict__ desc) {
-  const VecMove d = desc[blockIdx.y];
+constexpr int kMovesPerLaunch = 96;   // 3 KB of kernel arguments
+struct MoveArgs {
+  VecMove d[kMovesPerLaunch];
+};
+
+__global__ void move_batch_kernel(const MoveArgs args) {
+  const VecMove d = args.d[blockIdx.y];
   long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   const long long stride = (long long)gridDim.x * blockDim.x;
   switch (d.mode) {
@@ -136,25 +141,37 @@ __global__ void axpy_dev_kernel(double* __restrict__ y, const double* __restrict
   for (; i < n; i += stride) y[i] += av * x[i];
 }
 
-constexpr int kAxpyChunk = 4096;   // elements of one descriptor per workgroup
+constexpr int kAxpyChunk = 1024;   // elements of one group per workgroup
 
+// nsum consecutive descriptors from desc on (the bundle kernel's chunks name
+// one descriptor, and how it is walked in nsum)
 struct AxpyChunk {
-  int desc, first, count, pad;
+  int desc, first, count, nsum;
 };
 
-// One workgroup per chunk: elements [first, first + count) of one descriptor
-// in column-major order (r fastest), so the source reads coalesce.
+// One workgroup per chunk: elements [first, first + count) of one group in
+// column-major order (r fastest), so the source reads coalesce.  Bound by the
+// launch and the latency of its few loads at every size a step has; hence few
+// launches with small chunks.
 __global__ __launch_bounds__(kThreads) void strided_axpy_kernel(
     const StridedAxpy* __restrict__ desc, const AxpyChunk* __restrict__ chunks) {
   const AxpyChunk ch = chunks[blockIdx.x];
-  const StridedAxpy d = desc[ch.desc];
-  const int rows = d.rows;
+  const StridedAxpy* d = desc + ch.desc;
+  const int rows = d->rows;
+  const long long rs = d->rs, cs = d->cs;
   for (int j = threadIdx.x; j < ch.count; j += kThreads) {
     const int i = ch.first + j;
     const int c = i / rows, r = i - c * rows;
-    // a null source adds alpha (an identity block when rs/cs walk a diagonal)
-    double* p = d.dst + (r * d.rs + c * d.cs);
-    *p += d.src ? d.alpha * d.src[r + c * d.ld] : d.alpha;
+    double* p = d->dst + (r * rs + c * cs);
+    double acc = *p;
+    // rounded product, then the sum (not fused); a null source adds alpha (an
+    // identity block when rs/cs walk a diagonal)
+    for (int s = 0; s < ch.nsum; ++s) {
+#pragma clang fp contract(off)
+      const double v = d[s].src ? d[s].alpha * d[s].src[r + c * d[s].ld] : d[s].alpha;
+      acc += v;
+    }
+    *p = acc;
   }
 }
 
@@ -162,17 +179,17 @@ constexpr int kGatherChunk = 4096;   // bundle elements per workgroup
 
 constexpr int kGatherMaxPos = 16;    // summands held in registers (q-chunks)
 
-// A chunk is either elements [first, first + count) of the bundle (pad 0) or,
+// A chunk is either elements [first, first + count) of the bundle (nsum 0) or,
 // for an interleaved bundle of at most kThreads terms and kGatherMaxPos
 // summands, source positions q in [first, first + count) of every term
-// (pad 1): each thread then keeps one term, its sources and couplings in
+// (nsum 1): each thread then keeps one term, its sources and couplings in
 // registers, and walks q; lanes still write consecutive elements.
 __global__ __launch_bounds__(kThreads) void bundle_gather_kernel(
     const BundleDesc* __restrict__ desc, const BundleSrc* __restrict__ table,
     const AxpyChunk* __restrict__ chunks) {
   const AxpyChunk ch = chunks[blockIdx.x];
   const BundleDesc d = desc[ch.desc];
-  if (ch.pad) {
+  if (ch.nsum) {
     const int nt = d.nt, G = kThreads / nt;
     const int i = threadIdx.x;
     if (i >= G * nt) return;   // no barrier follows
@@ -215,7 +232,7 @@ __global__ __launch_bounds__(kThreads) void bundle_gather_kernel(
 }
 
 struct TileRef {
-  int desc, r0, c0, pad;
+  int desc, r0, c0, nsum;
 };
 
 constexpr int kTile = 64;
@@ -241,31 +258,41 @@ __global__ __launch_bounds__(kThreads) void transpose_kernel(const TransposeDesc
   }
 }
 
-// Strided scale-add of a descriptor that writes along its columns (cs == 1,
-// rs > 1): a 64 x 64 tile is read along r into LDS and added along c, so
-// both the reads and the writes coalesce.
+// Strided scale-adds of a group that writes along its columns (cs == 1,
+// rs > 1): 64 x 64 tiles are read along r, scaled and summed in registers onto
+// what is read from the destination along c through LDS, so that reads and
+// writes both coalesce.
 __global__ __launch_bounds__(kThreads) void strided_axpy_tiled_kernel(
     const StridedAxpy* __restrict__ desc, const TileRef* __restrict__ tiles) {
   __shared__ double t[kTile][kTile + 1];
   const TileRef tr = tiles[blockIdx.x];
-  const StridedAxpy d = desc[tr.desc];
+  const StridedAxpy* d = desc + tr.desc;
+  const int rows = d->rows, cols = d->cols;
   const int lx = threadIdx.x % kTile, ly = threadIdx.x / kTile;
   constexpr int kRowsPerPass = kThreads / kTile;
+  double* dst = d->dst;
+  const long long rs = d->rs;
+  for (int k = ly; k < kTile; k += kRowsPerPass) {
+    const int r = tr.r0 + k, c = tr.c0 + lx;
+    if (r < rows && c < cols) t[lx][k] = dst[r * rs + c];
+  }
+  __syncthreads();
   for (int k = ly; k < kTile; k += kRowsPerPass) {
     const int r = tr.r0 + lx, c = tr.c0 + k;
-    if (r < d.rows && c < d.cols) t[k][lx] = d.src[r + (long long)c * d.ld];
+    if (r >= rows || c >= cols) continue;
+    double acc = t[k][lx];
+    for (int s = 0; s < tr.nsum; ++s) {
+      // the arithmetic of strided_axpy_kernel
+#pragma clang fp contract(off)
+      const double v = d[s].alpha * d[s].src[r + (long long)c * d[s].ld];
+      acc += v;
+    }
+    t[k][lx] = acc;
   }
   __syncthreads();
   for (int k = ly; k < kTile; k += kRowsPerPass) {
     const int r = tr.r0 + k, c = tr.c0 + lx;
-    if (r < d.rows && c < d.cols) {
-      // rounded product, then the sum (not fused): the arithmetic of
-      // strided_axpy_kernel
-#pragma clang fp contract(off)
-      double* p = d.dst + (r * d.rs + c * d.cs);
-      const double v = d.alpha * t[lx][k];
-      *p += v;
-    }
+    if (r < rows && c < cols) dst[r * rs + c] = t[lx][k];
   }
 }
 
@@ -336,13 +363,20 @@ void dev_fill(Context& c, double* x, long long n, double v) {
   SU2_HIP(hipGetLastError());
 }
 
-void dev_move_batch(Context& c, const VecMove* d_desc, int ndesc, long long max_n) {
-  if (ndesc <= 0 || max_n <= 0) return;
-  SU2_CHECK(ndesc < 65536, kErrCapacity, "vector moves: %d descriptors", ndesc);
-  unsigned gx = grid_for(max_n);
-  if (gx > 1024) gx = 1024;
-  hipLaunchKernelGGL(move_batch_kernel, dim3(gx, ndesc), dim3(kThreads), 0, c.stream(), d_desc);
-  SU2_HIP(hipGetLastError());
+void dev_moves(Context& c, const std::vector<VecMove>& moves) {
+  MoveArgs args;
+  for (size_t i0 = 0; i0 < moves.size(); i0 += kMovesPerLaunch) {
+    const int n = (int)std::min<size_t>(kMovesPerLaunch, moves.size() - i0);
+    long long longest = 0;
+    for (int i = 0; i < n; ++i) {
+      args.d[i] = moves[i0 + i];
+      longest = std::max(longest, moves[i0 + i].n);
+    }
+    if (longest <= 0) continue;
+    const unsigned gx = std::min(1024u, grid_for(longest));
+    hipLaunchKernelGGL(move_batch_kernel, dim3(gx, n), dim3(kThreads), 0, c.stream(), args);
+    SU2_HIP(hipGetLastError());
+  }
 }
 
 void dev_fill_f32(Context& c, float* x, long long n, float v) {
@@ -427,7 +461,7 @@ void dev_axpy_dev(Context& c, double* y, const double* x, long long n, const dou
 }
 
 void dev_strided_axpy_launches(Context& c,
-                               const std::vector<std::vector<StridedAxpy>>& launches) {
+                               const std::vector<std::vector<StridedSum>>& launches) {
   std::vector<StridedAxpy> flat;
   std::vector<AxpyChunk> chunks;
   std::vector<TileRef> tiles;
@@ -435,18 +469,20 @@ void dev_strided_axpy_launches(Context& c,
   std::vector<std::pair<size_t, size_t>> span, tspan;
   for (auto& l : launches) {
     const size_t c0 = chunks.size(), t0 = tiles.size();
-    for (const StridedAxpy& d : l) {
+    for (const StridedSum& g : l) {
+      if (g.empty()) continue;
+      const StridedAxpy& d = g[0];
       const long long n = (long long)d.rows * d.cols;
       if (n <= 0) continue;
       SU2_CHECK(n < (1LL << 31), kErrCapacity, "strided axpy: block of %lld elements", n);
-      const int di = (int)flat.size();
-      flat.push_back(d);
+      const int di = (int)flat.size(), ns = (int)g.size();
+      flat.insert(flat.end(), g.begin(), g.end());
       if (d.src && d.cs == 1 && d.rs > 1 && d.rows > 1 && d.cols > 1) {
         for (int cc = 0; cc < d.cols; cc += kTile)
-          for (int r0 = 0; r0 < d.rows; r0 += kTile) tiles.push_back(TileRef{di, r0, cc, 0});
+          for (int r0 = 0; r0 < d.rows; r0 += kTile) tiles.push_back(TileRef{di, r0, cc, ns});
       } else {
         for (long long f = 0; f < n; f += kAxpyChunk)
-          chunks.push_back(AxpyChunk{di, (int)f, (int)std::min<long long>(kAxpyChunk, n - f), 0});
+          chunks.push_back(AxpyChunk{di, (int)f, (int)std::min<long long>(kAxpyChunk, n - f), ns});
       }
     }
     span.push_back({c0, chunks.size()});
@@ -468,7 +504,7 @@ void dev_strided_axpy_launches(Context& c,
   const StridedAxpy* d_desc = (const StridedAxpy*)dev;
   const AxpyChunk* d_chunks = (const AxpyChunk*)(dev + dbytes);
   const TileRef* d_tiles = (const TileRef*)(dev + dbytes + cbytes);
-  // the descriptors of one launch write disjoint elements, so its chunked
+  // the groups of one launch write disjoint elements, so its chunked
   // and tiled parts may run in either order
   for (size_t i = 0; i < span.size(); ++i) {
     const auto& s = span[i];
@@ -485,10 +521,6 @@ void dev_strided_axpy_launches(Context& c,
     }
   }
   c.dev_free(dev);
-}
-
-void dev_strided_axpy(Context& c, const std::vector<StridedAxpy>& desc) {
-  dev_strided_axpy_launches(c, {desc});
 }
 
 }  // namespace su2

@@ -16,10 +16,9 @@ class Context;
 
 void dev_fill(Context& c, double* x, long long n, double v);
 void dev_copy(Context& c, double* y, const double* x, long long n);
-// Many vector moves in one launch (descriptors in device memory, ndesc of
-// them, the longest max_n elements): copies, FP64 -> FP32 rounding, FP32 ->
-// FP64 widening, zero fills.  Used by the batched H_eff apply, whose launch
-// sequence is captured in a HIP graph (a fill kernel, never a memset node).
+// Many vector moves in a launch, the descriptors as kernel arguments (nothing
+// to upload, and a captured launch keeps them): copies, FP64 -> FP32 rounding,
+// FP32 -> FP64 widening, zero fills (a fill kernel, never a memset node).
 enum VecMoveMode : int { kMoveF64 = 0, kMoveF64toF32 = 1, kMoveF32toF64 = 2, kZeroF64 = 3,
                          kZeroF32 = 4 };
 struct VecMove {
@@ -28,7 +27,7 @@ struct VecMove {
   long long n;
   int mode, pad;
 };
-void dev_move_batch(Context& c, const VecMove* d_desc, int ndesc, long long max_n);
+void dev_moves(Context& c, const std::vector<VecMove>& moves);
 // FP32 buffers of the mixed-precision matvec: fill, round to FP32, widen
 void dev_fill_f32(Context& c, float* x, long long n, float v);
 void dev_convert_f64_f32(Context& c, float* y, const double* x, long long n);
@@ -64,13 +63,16 @@ struct StridedAxpy {
   int rows, cols;   // rows * cols < 2^31
   double alpha;
 };
-// One launch per inner vector, in order on the context stream (a later
-// launch may add into what an earlier one wrote); the descriptors of all
-// launches are uploaded together and the call does not wait.  Every descriptor
-// is cut into chunks of up to 4096 elements, one workgroup each, so a
-// workgroup reads its descriptor once and indexes with 32-bit arithmetic.
-void dev_strided_axpy_launches(Context& c, const std::vector<std::vector<StridedAxpy>>& launches);
-void dev_strided_axpy(Context& c, const std::vector<StridedAxpy>& desc);
+// Descriptors of one group share destination, strides and shape (and whether
+// they have a source); their terms are added one after the other, in order.
+typedef std::vector<StridedAxpy> StridedSum;
+// One launch per inner vector of groups, in order on the context stream (a
+// later launch may add into what an earlier one wrote); the descriptors of
+// all launches are uploaded together and the call does not wait.  Every group
+// is cut into chunks of up to kAxpyChunk elements, one workgroup each, so a
+// workgroup reads its descriptors once and indexes with 32-bit arithmetic,
+// and an element is read and written once however many terms it has.
+void dev_strided_axpy_launches(Context& c, const std::vector<std::vector<StridedSum>>& launches);
 
 // Operator bundles: each descriptor holds nt summands of rows x cols
 // column-major blocks, element q = r + rows*c of summand t written once as

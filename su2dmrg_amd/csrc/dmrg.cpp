@@ -458,7 +458,8 @@ std::unique_ptr<Dmrg::Solve> Dmrg::prepare(int il, int ir, std::unique_ptr<Tenso
 
   t0 = now();
   S.t_lanczos0 = t0;
-  S.psi.reset(new Tensor(&c, {with_dir(o.FL.fused, 1), with_dir(o.FR.fused, 1)}, 0, nullptr));
+  S.psi.reset(
+      new Tensor(&c, {with_dir(o.FL.fused, 1), with_dir(o.FR.fused, 1)}, 0, nullptr, false));
   SU2_CHECK(S.psi->size() > 0, kErrStructure, "step %d,%d: no common sector for spin %d", il, ir,
             S_);
   if (psi0) {

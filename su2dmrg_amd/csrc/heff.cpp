@@ -166,7 +166,6 @@ HeffPlan::HeffPlan(Context& c, const Tensor& psi, const Tensor* hl, const Tensor
   d_in_ = c.dev_alloc_n<double>(std::max<long long>(psi_size_, 1));
   d_out_ = c.dev_alloc_n<double>(std::max<long long>(psi_size_, 1));
   if (work > 0) d_work_ = c.dev_alloc_n<double>(work);
-  dev_fill(c, d_work_, work, 0.0);
 
   // bundle assembly: each bundle element is the sum of its coupling's
   // summands in the order given (deterministic), written once; then H_L of
@@ -209,10 +208,12 @@ HeffPlan::HeffPlan(Context& c, const Tensor& psi, const Tensor* hl, const Tensor
     transposes.push_back(TransposeDesc{d_work_ + kv.second, hl->data() + hb.offset, hb.dim[0]});
   }
   dev_transpose_batch(c, transposes);
+  std::vector<VecMove> copies;
   for (auto& kv : hr_off) {
     const Block& hb = hr->blocks()[hr->find2(kv.first, kv.first)];
-    dev_copy(c, d_work_ + kv.second, hr->data() + hb.offset, hb.size);
+    copies.push_back(VecMove{hr->data() + hb.offset, d_work_ + kv.second, hb.size, kMoveF64, 0});
   }
+  dev_moves(c, copies);
 
   // The two launches as problems over three buffers (bundle workspace, input,
   // output) with element offsets, instantiated for FP64 now and for FP32

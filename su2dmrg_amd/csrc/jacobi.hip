@@ -2,6 +2,7 @@
 #include "jacobi.hpp"
 
 #include <algorithm>
+#include <functional>
 #include <map>
 #include <cmath>
 #include <cstring>
@@ -960,23 +961,29 @@ __global__ __launch_bounds__(SolveThreads<CB>::value) void apply_kernel(
 // Largest overlap that calls for a rotation in each pair of column blocks (i
 // <= j) of a block's kept columns, from their whole Gram matrix (0: none);
 // workgroup = entry of the pair table.
-struct FlagJob {
-  const double* G;   // kept x kept, ld ldg
-  int ldg, kept, i, j;
+struct FlagBlock {
+  const double* G;   // kept x kept
+  int kept, first;   // its pairs of column blocks (i <= j, row by row) from workgroup `first` on
   double normF;
 };
 
-__global__ __launch_bounds__(256) void pair_flags_kernel(const FlagJob* __restrict__ jobs, int cb,
-                                                         double tol_rel, double tol_abs,
-                                                         double* __restrict__ out) {
+__global__ __launch_bounds__(256) void pair_flags_kernel(const FlagBlock* __restrict__ blocks,
+                                                         int nblocks, int cb, double tol_rel,
+                                                         double tol_abs, double* __restrict__ out) {
   __shared__ double s[4];
-  const FlagJob J = jobs[blockIdx.x];
+  int b = nblocks - 1;
+  while (b > 0 && blocks[b].first > (int)blockIdx.x) --b;
+  const FlagBlock J = blocks[b];
+  const int ncb = (J.kept + cb - 1) / cb;
+  int i = 0, f = (int)blockIdx.x - J.first;
+  while (f >= ncb - i) f -= ncb - i++;
+  const int j = i + f;
   double worst = 0.0;
   for (int e = threadIdx.x; e < cb * cb; e += 256) {
-    const int a = J.i * cb + e % cb, b = J.j * cb + e / cb;
+    const int a = i * cb + e % cb, b = j * cb + e / cb;
     if (a >= b || b >= J.kept) continue;
-    const double ga = J.G[a + (size_t)a * J.ldg], gb = J.G[b + (size_t)b * J.ldg];
-    worst = fmax(worst, pair_overlap(J.G[a + (size_t)b * J.ldg], ga, gb, tol_rel, tol_abs,
+    const double ga = J.G[a + (size_t)a * J.kept], gb = J.G[b + (size_t)b * J.kept];
+    worst = fmax(worst, pair_overlap(J.G[a + (size_t)b * J.kept], ga, gb, tol_rel, tol_abs,
                                      J.normF));
   }
 #pragma unroll
@@ -986,92 +993,54 @@ __global__ __launch_bounds__(256) void pair_flags_kernel(const FlagJob* __restri
   if (threadIdx.x == 0) out[blockIdx.x] = fmax(fmax(s[0], s[1]), fmax(s[2], s[3]));
 }
 
-// W = A (transpose = 0) or A^T (transpose = 1); A is m x n with ld m
-__global__ void load_work_kernel(const double* __restrict__ A, int m, int n, int transpose,
-                                 double* __restrict__ W) {
+// Every block's start in one launch, blockIdx.y the block: W = A, or A^T where
+// A is wider than tall (m x n, ld m), in 32 x 32 tiles, and V = 1 in the rest
+// of the grid.
+struct LoadJob {
+  const double* A;
+  double *W, *V;
+  int m, n;
+};
+constexpr int kLoadsPerLaunch = 96;
+struct LoadArgs {
+  LoadJob j[kLoadsPerLaunch];
+};
+
+__global__ __launch_bounds__(256) void load_kernel(const LoadArgs args) {
   __shared__ double tile[32][33];
-  const int bx = blockIdx.x * 32, by = blockIdx.y * 32;
-  const int tx = threadIdx.x, ty = threadIdx.y;   // 32 x 8
-  if (!transpose) {
+  const LoadJob J = args.j[blockIdx.y];
+  const int m = J.m, n = J.n, tm = (m + 31) / 32, tn = (n + 31) / 32;
+  const int tx = threadIdx.x % 32, ty = threadIdx.x / 32;   // 32 x 8
+  if ((int)blockIdx.x >= tm * tn) {
+    const int k = min(m, n);
+    const long long e0 = ((long long)blockIdx.x - tm * tn) * 1024;
+    for (long long e = e0 + threadIdx.x; e < min(e0 + 1024, (long long)k * k); e += 256)
+      J.V[e] = (e % k) == (e / k) ? 1.0 : 0.0;
+    return;
+  }
+  const int bx = (int)blockIdx.x % tm * 32, by = (int)blockIdx.x / tm * 32;
+  if (m >= n) {
     for (int j = ty; j < 32; j += 8) {
       const int r = bx + tx, c = by + j;
-      if (r < m && c < n) W[r + (long long)c * m] = A[r + (long long)c * m];
+      if (r < m && c < n) J.W[r + (long long)c * m] = J.A[r + (long long)c * m];
     }
     return;
   }
   // W (n x m) = A^T: read A tile (rows bx.., cols by..), write transposed
   for (int j = ty; j < 32; j += 8) {
     const int r = bx + tx, c = by + j;
-    tile[j][tx] = (r < m && c < n) ? A[r + (long long)c * m] : 0.0;
+    tile[j][tx] = (r < m && c < n) ? J.A[r + (long long)c * m] : 0.0;
   }
   __syncthreads();
   for (int j = ty; j < 32; j += 8) {
     const int wr = by + tx, wc = bx + j;   // W row = A column, W column = A row
-    if (wr < n && wc < m) W[wr + (long long)wc * n] = tile[tx][j];
+    if (wr < n && wc < m) J.W[wr + (long long)wc * n] = tile[tx][j];
   }
-}
-
-__global__ void eye_kernel(double* __restrict__ V, int k) {
-  const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e < (long long)k * k) V[e] = (e % k) == (e / k) ? 1.0 : 0.0;
-}
-
-// squared column norms of W (one workgroup per column)
-__global__ __launch_bounds__(256) void colnorm_kernel(const double* __restrict__ W, int L,
-                                                      double* __restrict__ out) {
-  __shared__ double s[256];
-  const double* col = W + (long long)blockIdx.x * L;
-  double a = 0.0;
-  for (int r = threadIdx.x; r < L; r += 256) a += col[r] * col[r];
-  s[threadIdx.x] = a;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) out[blockIdx.x] = s[0];
-}
-
-// dst[:, c] = sign[c] * src[:, perm[c]]
-__global__ void permute_cols_kernel(const double* __restrict__ src, double* __restrict__ dst,
-                                    const int* __restrict__ perm, const double* __restrict__ sign,
-                                    int rows, int cols) {
-  const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= (long long)rows * cols) return;
-  const int r = (int)(e % rows), c = (int)(e / rows);
-  dst[e] = sign[c] * src[r + (long long)perm[c] * rows];
 }
 
 __global__ void fill_u64_kernel(unsigned long long* __restrict__ p, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = 0ull;
-}
-
-// sign of the first entry with |v| >= max|v|/2 of each column (as +-1)
-__global__ __launch_bounds__(256) void col_sign_kernel(const double* __restrict__ V, int rows,
-                                                       double* __restrict__ sign) {
-  __shared__ double sv[256];
-  __shared__ int si[256];
-  const double* col = V + (long long)blockIdx.x * rows;
-  double best = 0.0;
-  for (int r = threadIdx.x; r < rows; r += 256) best = fmax(best, fabs(col[r]));
-  sv[threadIdx.x] = best;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) sv[threadIdx.x] = fmax(sv[threadIdx.x], sv[threadIdx.x + w]);
-    __syncthreads();
-  }
-  const double half = 0.5 * sv[0];
-  int first = 0x7fffffff;
-  for (int r = threadIdx.x; r < rows; r += 256)
-    if (fabs(col[r]) >= half && r < first) first = r;
-  si[threadIdx.x] = first;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) si[threadIdx.x] = min(si[threadIdx.x], si[threadIdx.x + w]);
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) sign[blockIdx.x] = (si[0] < rows && col[si[0]] < 0.0) ? -1.0 : 1.0;
 }
 
 // ---- batched helpers: one launch for every block of the batch ----
@@ -1141,23 +1110,27 @@ __global__ void permute_batched_kernel(const PermJob* __restrict__ jobs, int nj,
   const PermJob J = jobs[lo];
   const long long i = e - J.elem_begin;
   const int r = (int)(i % J.rows), c = (int)(i / J.rows);
-  J.dst[i] = sign[J.col_off + c] * J.src[r + (long long)perm[J.col_off + c] * J.rows];
+  const double v = J.src[r + (long long)perm[J.col_off + c] * J.rows];
+  J.dst[i] = sign ? sign[J.col_off + c] * v : v;
 }
 
-// col_sign_kernel for the V of every block (desc[b].V, k x k), divided by
+// Sign of the first entry with |v| >= max|v|/2 of the columns perm[] of every
+// block's V (desc[b].V, k x k), divided by
 // the column's norm: the accumulated rotations leave V's columns off unit
 // length by the rounding of every rotation applied (a few 1e-13 after tens of
 // sweeps over hundreds of columns), and W = A V carries the same factor, so
 // one scaling of both restores the triplet
 __global__ __launch_bounds__(256) void col_sign_batched_kernel(const BlockDesc* __restrict__ desc,
                                                                const long long* __restrict__ noff,
-                                                               int nb, double* __restrict__ sign) {
+                                                               int nb,
+                                                               const int* __restrict__ perm,
+                                                               double* __restrict__ sign) {
   __shared__ double sv[256];
   __shared__ int si[256];
   const long long gc = blockIdx.x;
   const int b = col_block(noff, nb, gc);
   const int rows = desc[b].k;
-  const double* col = desc[b].V + (gc - noff[b]) * rows;
+  const double* col = desc[b].V + (long long)perm[gc] * rows;
   double best = 0.0;
   for (int r = threadIdx.x; r < rows; r += 256) best = fmax(best, fabs(col[r]));
   sv[threadIdx.x] = best;
@@ -1242,58 +1215,82 @@ static int jacobi_svd_large(Context& c, const std::vector<JacobiBlock*>& blocks,
     Vc[b] = J.V;
     Wo[b] = (double*)W2[b]->p;
     Vo[b] = (double*)V2[b]->p;
-    hipLaunchKernelGGL(load_work_kernel, dim3(nblk(J.m, 32), nblk(J.n, 32)), dim3(32, 8), 0, st,
-                       J.A, J.m, J.n, J.m < J.n ? 1 : 0, J.W);
-    hipLaunchKernelGGL(eye_kernel, dim3(nblk((long long)K[b] * K[b], 256)), dim3(256), 0, st, J.V,
-                       K[b]);
   }
-  SU2_HIP(hipGetLastError());
-  DevMem dn(c, sizeof(double) * 2 * ncol), dperm(c, sizeof(int) * ncol),
-      done(c, sizeof(double) * ncol), dsign(c, sizeof(double) * ncol),
-      dnoff(c, sizeof(long long) * (nb + 1)), dpj(c, sizeof(PermJob) * 2 * nb);
+  for (int b0 = 0; b0 < nb; b0 += kLoadsPerLaunch) {
+    LoadArgs args;
+    const int n = std::min(kLoadsPerLaunch, nb - b0);
+    long long most = 1;
+    for (int i = 0; i < n; ++i) {
+      const JacobiBlock& J = *blocks[b0 + i];
+      args.j[i] = LoadJob{J.A, J.W, J.V, J.m, J.n};
+      const long long k = K[b0 + i];
+      most = std::max(most, (long long)nblk(J.m, 32) * nblk(J.n, 32) + nblk(k * k, 1024));
+    }
+    hipLaunchKernelGGL(load_kernel, dim3((unsigned)most, n), dim3(256), 0, st, args);
+    SU2_HIP(hipGetLastError());
+  }
+  // The tables that change from sweep to sweep, [permutation jobs | blocks |
+  // flag blocks | permutation], in one device block and one upload.  A copy of
+  // any size costs the host 3 us and the stream as much, and one back through
+  // pageable memory 20 us with its wait, where a kernel that writes to pinned
+  // memory needs 11: with one upload here, norms and flags written to pinned
+  // memory, and descriptors as kernel arguments wherever a table goes to one
+  // launch, a 6x4 lattice run up to d = 924 went from 310 to 262 ms, eight
+  // small jobs from 341 to 262, a truncation at 64 multiplets from 0.47 to
+  // 0.36 ms and one at 500 from 9.2 to 8.3.
+  const size_t off_desc = sizeof(PermJob) * 2 * nb, off_flag = off_desc + sizeof(BlockDesc) * nb,
+               off_perm = off_flag + sizeof(FlagBlock) * nb;
+  DevMem dtab(c, off_perm + sizeof(int) * ncol), dsign(c, sizeof(double) * ncol),
+      dnoff(c, sizeof(long long) * (nb + 1));
+  std::vector<char> tab(off_perm + sizeof(int) * ncol, 0);
+  PermJob* const hpj = (PermJob*)tab.data();
+  FlagBlock* const hflag = (FlagBlock*)(tab.data() + off_flag);
+  int* const hp = (int*)(tab.data() + off_perm);
+  const PermJob* const dpj = (const PermJob*)dtab.p;
+  const BlockDesc* const ddesc = (const BlockDesc*)((char*)dtab.p + off_desc);
+  const FlagBlock* const dflagb = (const FlagBlock*)((char*)dtab.p + off_flag);
+  const int* const dperm = (const int*)((char*)dtab.p + off_perm);
   std::vector<double> hn(2 * ncol);   // W then V squared column norms
-  std::vector<int> hp(ncol);
-  {
-    std::vector<double> ones(ncol, 1.0);
-    SU2_HIP(hipMemcpyAsync(done.p, ones.data(), sizeof(double) * ncol, hipMemcpyHostToDevice, st));
-    SU2_HIP(hipMemcpyAsync(dnoff.p, noff.data(), sizeof(long long) * (nb + 1),
-                           hipMemcpyHostToDevice, st));
-  }
+  SU2_HIP(hipMemcpyAsync(dnoff.p, noff.data(), sizeof(long long) * (nb + 1), hipMemcpyHostToDevice,
+                         st));
   std::vector<BlockDesc> desc(nb);
-  DevMem ddesc(c, sizeof(BlockDesc) * nb);
-  auto upload_desc = [&]() {
+  auto upload = [&]() {
     for (int b = 0; b < nb; ++b) {
       desc[b].W = Wc[b];
       desc[b].V = Vc[b];
     }
-    SU2_HIP(hipMemcpyAsync(ddesc.p, desc.data(), sizeof(BlockDesc) * nb, hipMemcpyHostToDevice,
-                           st));
+    std::memcpy(tab.data() + off_desc, desc.data(), sizeof(BlockDesc) * nb);
+    SU2_HIP(hipMemcpyAsync(dtab.p, tab.data(), tab.size(), hipMemcpyHostToDevice, st));
   };
-  // squared column norms of the current W of every block, to the host
+  // squared column norms of the current W and V of every block, written to
+  // pinned memory by the kernel
   auto norms = [&]() {
-    hipLaunchKernelGGL(colnorm_batched_kernel, dim3((unsigned)ncol), dim3(256), 0, st,
-                       (const BlockDesc*)ddesc.p, (const long long*)dnoff.p, nb, (long long)ncol,
-                       (double*)dn.p);
-    SU2_HIP(hipMemcpyAsync(hn.data(), dn.p, sizeof(double) * 2 * ncol, hipMemcpyDeviceToHost,
-                           st));
+    double* h = c.host_scratch(2 * ncol);
+    hipLaunchKernelGGL(colnorm_batched_kernel, dim3((unsigned)ncol), dim3(256), 0, st, ddesc,
+                       (const long long*)dnoff.p, nb, (long long)ncol, h);
+    SU2_HIP(hipGetLastError());
     SU2_HIP(hipStreamSynchronize(st));
+    std::memcpy(hn.data(), h, sizeof(double) * 2 * ncol);
   };
-  // src -> dst column moves of W and V (or the given jobs) in one launch
-  auto permute = [&](const std::vector<PermJob>& pj0, const double* sign) {
-    std::vector<PermJob> pj = pj0;
-    long long tot = 0;
-    for (auto& j : pj) {
-      j.elem_begin = tot;
-      tot += (long long)j.rows * j.cols;
+  // src -> dst column moves of W and V: the first n jobs of the table
+  // (prepare_permute before the upload, permute after it)
+  long long perm_total = 0;
+  auto prepare_permute = [&](const std::vector<PermJob>& pj) {
+    perm_total = 0;
+    for (size_t i = 0; i < pj.size(); ++i) {
+      hpj[i] = pj[i];
+      hpj[i].elem_begin = perm_total;
+      perm_total += (long long)pj[i].rows * pj[i].cols;
     }
-    if (tot == 0) return;
-    SU2_HIP(hipMemcpyAsync(dpj.p, pj.data(), sizeof(PermJob) * pj.size(), hipMemcpyHostToDevice,
-                           st));
-    hipLaunchKernelGGL(permute_batched_kernel, dim3(nblk(tot, 256)), dim3(256), 0, st,
-                       (const PermJob*)dpj.p, (int)pj.size(), tot, (const int*)dperm.p, sign);
+  };
+  auto permute = [&](int n, const double* sign) {
+    if (perm_total == 0) return;
+    hipLaunchKernelGGL(permute_batched_kernel, dim3(nblk(perm_total, 256)), dim3(256), 0, st, dpj,
+                       n, perm_total, dperm, sign);
+    SU2_HIP(hipGetLastError());
   };
   for (int b = 0; b < nb; ++b) desc[b] = BlockDesc{Wc[b], Vc[b], L[b], K[b], 0.0};
-  upload_desc();
+  upload();
   norms();
   for (int b = 0; b < nb; ++b) {
     double g = 0;
@@ -1306,12 +1303,12 @@ static int jacobi_svd_large(Context& c, const std::vector<JacobiBlock*>& blocks,
   // rotation (later sweeps would leave it unchanged: its columns stay in
   // order and no pair rotates), so converged blocks cost no further rounds
   std::vector<char> active(nb, 1);
-  auto sort_permute = [&]() {
+  auto sort_permute = [&](const std::function<bool()>& tables) {
     std::vector<PermJob> pj;
     std::vector<char> moved(nb, 0);
     for (int b = 0; b < nb; ++b) {
       if (!active[b]) continue;
-      int* p = hp.data() + noff[b];
+      int* p = hp + noff[b];
       const double* w = hn.data() + noff[b];
       std::iota(p, p + K[b], 0);
       std::stable_sort(p, p + K[b], [&](int x, int y) { return w[x] > w[y]; });
@@ -1325,15 +1322,17 @@ static int jacobi_svd_large(Context& c, const std::vector<JacobiBlock*>& blocks,
       pj.push_back(PermJob{Wc[b], Wo[b], L[b], K[b], 0, noff[b]});
       pj.push_back(PermJob{Vc[b], Vo[b], K[b], K[b], 0, noff[b]});
     }
-    if (pj.empty()) return;
-    SU2_HIP(hipMemcpyAsync(dperm.p, hp.data(), sizeof(int) * ncol, hipMemcpyHostToDevice, st));
-    permute(pj, (const double*)done.p);
     for (int b = 0; b < nb; ++b) {
       if (!moved[b]) continue;
       std::swap(Wc[b], Wo[b]);
       std::swap(Vc[b], Vo[b]);
     }
-    upload_desc();
+    // the caller's entries that follow from the order
+    const bool more = tables && tables();
+    if (pj.empty() && !more) return;
+    prepare_permute(pj);
+    upload();
+    permute((int)pj.size(), nullptr);
   };
   // QR preconditioning (precond.hpp) of every block with precondition_min_k
   // <= K <= kPrecondMaxK: columns sorted, then W <- W P Q2 and V <- P Q2.  A block's
@@ -1349,7 +1348,7 @@ static int jacobi_svd_large(Context& c, const std::vector<JacobiBlock*>& blocks,
         pre.push_back(b);
       }
     if (!pre.empty()) {
-      sort_permute();
+      sort_permute(nullptr);
       for (int b : pre)
         pb.push_back(PrecondBlock{Wc[b], Vc[b], Wo[b], Vo[b], L[b], K[b], K[b], desc[b].normF, 0.0});
       precondition_jacobi(c, pb);
@@ -1357,14 +1356,14 @@ static int jacobi_svd_large(Context& c, const std::vector<JacobiBlock*>& blocks,
         std::swap(Wc[b], Wo[b]);
         std::swap(Vc[b], Vo[b]);
       }
-      upload_desc();
+      upload();
       norms();
       // The Gram matrix resolves directions down to 3e-8 of the block; the
       // columns below that are still a mixture of everything under it.
       // They are preconditioned among themselves, with their own Gram matrix
       // (which resolves 3e-8 of theirs), so that the null space drops to the
       // rounding level at once and leaves the sweeps.
-      if (!plain) sort_permute();
+      if (!plain) sort_permute(nullptr);
       std::vector<PrecondBlock> tail;
       std::vector<VecMove> back;
       for (const int b : plain ? std::vector<int>() : pre) {
@@ -1388,12 +1387,7 @@ static int jacobi_svd_large(Context& c, const std::vector<JacobiBlock*>& blocks,
       }
       if (!tail.empty()) {
         precondition_jacobi(c, tail);
-        long long mx = 0;
-        for (auto& m : back) mx = std::max(mx, m.n);
-        DevMem dm(c, sizeof(VecMove) * back.size());
-        SU2_HIP(hipMemcpyAsync(dm.p, back.data(), sizeof(VecMove) * back.size(),
-                               hipMemcpyHostToDevice, st));
-        dev_move_batch(c, (const VecMove*)dm.p, (int)back.size(), mx);
+        dev_moves(c, back);
       }
       if (!tail.empty()) norms();
     }
@@ -1505,7 +1499,7 @@ static int jacobi_svd_large(Context& c, const std::vector<JacobiBlock*>& blocks,
       ++sweeps_done;
       // descending column norms (hn: read back with the previous sweep's
       // convergence counters, or before the first sweep)
-      sort_permute();
+      sort_permute(nullptr);
       hipLaunchKernelGGL(fill_u64_kernel, dim3(nblk(nb, 256)), dim3(256), 0, st,
                          (unsigned long long*)doff.p, nb);
       for (size_t r = 0; r < rounds.size(); ++r) {
@@ -1515,16 +1509,16 @@ static int jacobi_svd_large(Context& c, const std::vector<JacobiBlock*>& blocks,
         const PairJob* jr = (const PairJob*)djobs.p + round_off[r];
         if (CB == 16) {
           hipLaunchKernelGGL((gram_partial_kernel<16, 64, RCH>), dim3(nj * pm), dim3(64), 0, st,
-                             (const BlockDesc*)ddesc.p, jr, pm, (double*)dgpart.p);
+                             ddesc, jr, pm, (double*)dgpart.p);
           hipLaunchKernelGGL((jacobi_rotate_kernel<16, 64>), dim3(nj * pm), dim3(64), 0, st,
-                             (const BlockDesc*)ddesc.p, jr, pm, (const double*)dgpart.p, tol,
+                             ddesc, jr, pm, (const double*)dgpart.p, tol,
                              kTolAbs,
                              (unsigned long long*)doff.p, inner_sweeps);
         } else {
           hipLaunchKernelGGL((gram_partial_kernel<32, 1024, 64>), dim3(nj * pm), dim3(1024), 0, st,
-                             (const BlockDesc*)ddesc.p, jr, pm, (double*)dgpart.p);
+                             ddesc, jr, pm, (double*)dgpart.p);
           hipLaunchKernelGGL((jacobi_rotate_kernel<32, 512>), dim3(nj * pm), dim3(512), 0, st,
-                             (const BlockDesc*)ddesc.p, jr, pm, (const double*)dgpart.p, tol,
+                             ddesc, jr, pm, (const double*)dgpart.p, tol,
                              kTolAbs,
                              (unsigned long long*)doff.p, inner_sweeps);
         }
@@ -1534,12 +1528,7 @@ static int jacobi_svd_large(Context& c, const std::vector<JacobiBlock*>& blocks,
                              hipMemcpyDeviceToHost, st));
       // the column norms for the next sweep's order (or the final one) come
       // back with the counters: one wait per sweep
-      hipLaunchKernelGGL(colnorm_batched_kernel, dim3((unsigned)ncol), dim3(256), 0, st,
-                         (const BlockDesc*)ddesc.p, (const long long*)dnoff.p, nb, (long long)ncol,
-                         (double*)dn.p);
-      SU2_HIP(hipMemcpyAsync(hn.data(), dn.p, sizeof(double) * 2 * ncol, hipMemcpyDeviceToHost,
-                             st));
-      SU2_HIP(hipStreamSynchronize(st));
+      norms();
       converged = true;
       worst = 0;
       bool left = false;
@@ -1571,34 +1560,39 @@ static int jacobi_svd_large(Context& c, const std::vector<JacobiBlock*>& blocks,
     std::vector<std::unique_ptr<DevMem>> gram(nb);
     for (int b = 0; b < nb; ++b)
       gram[b].reset(new DevMem(c, sizeof(double) * (size_t)K[b] * K[b]));
+    // flag blocks of the table: how many, their pairs, each block's first pair
+    int nflag = 0, npair = 0;
+    std::vector<size_t> f0(nb, 0);
+    auto flag_blocks = [&]() {
+      count_kept();
+      nflag = npair = 0;
+      for (int b = 0; b < nb; ++b) {
+        f0[b] = npair;
+        if (!active[b] || kept[b] < 2) continue;
+        const int ncb = (kept[b] + CB - 1) / CB;
+        hflag[nflag++] = FlagBlock{(const double*)gram[b]->p, kept[b], npair, desc[b].normF};
+        npair += ncb * (ncb + 1) / 2;
+      }
+      return nflag > 0;
+    };
     auto build_schedule = [&]() {
       rounds.clear();
       all.clear();
-      std::vector<FlagJob> fj;
-      std::vector<size_t> f0(nb, 0);
       GemmBatch g;
       for (int b = 0; b < nb; ++b) {
-        if (!active[b]) continue;
-        const int kb = kept[b], ncb = (kb + CB - 1) / CB;
-        double* G = (double*)gram[b]->p;
-        f0[b] = fj.size();
-        if (kb < 2) continue;
-        g.add(G, kb, kb, kb, Wc[b], L[b], 1, Wc[b], L[b], 0, L[b]);
-        for (int i = 0; i < ncb; ++i)
-          for (int j = i; j < ncb; ++j) fj.push_back(FlagJob{G, kb, kb, i, j, desc[b].normF});
+        const int kb = kept[b];
+        if (!active[b] || kb < 2) continue;
+        g.add((double*)gram[b]->p, kb, kb, kb, Wc[b], L[b], 1, Wc[b], L[b], 0, L[b]);
       }
       g.run(c);
-      std::vector<double> flag(fj.size());
-      if (!fj.empty()) {
-        DevMem df(c, sizeof(FlagJob) * fj.size()), dflag(c, sizeof(double) * fj.size());
-        SU2_HIP(hipMemcpyAsync(df.p, fj.data(), sizeof(FlagJob) * fj.size(), hipMemcpyHostToDevice,
-                               st));
-        hipLaunchKernelGGL(pair_flags_kernel, dim3((unsigned)fj.size()), dim3(256), 0, st,
-                           (const FlagJob*)df.p, CB, tol, kTolAbs, (double*)dflag.p);
+      std::vector<double> flag(npair);
+      if (npair > 0) {
+        double* h = c.host_scratch(npair);
+        hipLaunchKernelGGL(pair_flags_kernel, dim3((unsigned)npair), dim3(256), 0, st, dflagb, nflag,
+                           CB, tol, kTolAbs, h);
         SU2_HIP(hipGetLastError());
-        SU2_HIP(hipMemcpyAsync(flag.data(), dflag.p, sizeof(double) * fj.size(),
-                               hipMemcpyDeviceToHost, st));
         SU2_HIP(hipStreamSynchronize(st));
+        std::memcpy(flag.data(), h, sizeof(double) * npair);
       }
       worst = 0;
       for (int b = 0; b < nb; ++b) {
@@ -1697,7 +1691,7 @@ static int jacobi_svd_large(Context& c, const std::vector<JacobiBlock*>& blocks,
     auto run_rounds = [&](auto cb) {
       constexpr int B = decltype(cb)::value;
       constexpr int NT = SolveThreads<B>::value;
-      const BlockDesc* dd = (const BlockDesc*)ddesc.p;
+      const BlockDesc* dd = ddesc;
       DevMem djobs(c, sizeof(PairJob) * all.size());
       SU2_HIP(hipMemcpyAsync(djobs.p, all.data(), sizeof(PairJob) * all.size(),
                              hipMemcpyHostToDevice, st));
@@ -1732,8 +1726,7 @@ static int jacobi_svd_large(Context& c, const std::vector<JacobiBlock*>& blocks,
     };
     for (int sweep = 0; sweep <= max_sweeps; ++sweep) {
       // descending column norms (hn: read back after the previous sweep)
-      sort_permute();
-      count_kept();
+      sort_permute(flag_blocks);
       build_schedule();
       converged = all.empty();
       if (converged || sweep == max_sweeps) break;
@@ -1756,7 +1749,6 @@ static int jacobi_svd_large(Context& c, const std::vector<JacobiBlock*>& blocks,
   // singular values in ascending order, sign convention on V (W follows),
   // results into the caller's buffers -- for every block in a few launches;
   // hn holds the final column norms
-  std::vector<int> ident(ncol);
   for (int b = 0; b < nb; ++b) {
     JacobiBlock& J = *blocks[b];
     const int k = K[b];
@@ -1766,58 +1758,31 @@ static int jacobi_svd_large(Context& c, const std::vector<JacobiBlock*>& blocks,
       const double v2 = hn[ncol + noff[b] + i];
       s2[i] = v2 > 0.0 ? hn[noff[b] + i] / v2 : hn[noff[b] + i];
     }
-    int* perm = hp.data() + noff[b];
+    int* perm = hp + noff[b];
     std::iota(perm, perm + k, 0);
-    std::iota(ident.data() + noff[b], ident.data() + noff[b] + k, 0);
     std::stable_sort(perm, perm + k, [&](int x, int y) { return s2[x] < s2[y]; });
     J.s.resize(k);
     for (int i = 0; i < k; ++i) J.s[i] = std::sqrt(s2[perm[i]]);
   }
-  DevMem dident(c, sizeof(int) * ncol);
-  SU2_HIP(hipMemcpyAsync(dperm.p, hp.data(), sizeof(int) * ncol, hipMemcpyHostToDevice, st));
-  SU2_HIP(hipMemcpyAsync(dident.p, ident.data(), sizeof(int) * ncol, hipMemcpyHostToDevice, st));
-  // V: sorted copy in the spare buffer, its signs
-  {
-    std::vector<PermJob> pj;
-    for (int b = 0; b < nb; ++b) pj.push_back(PermJob{Vc[b], Vo[b], K[b], K[b], 0, noff[b]});
-    permute(pj, (const double*)done.p);
-  }
-  for (int b = 0; b < nb; ++b) {
-    desc[b].W = Wc[b];
-    desc[b].V = Vo[b];
-  }
-  SU2_HIP(hipMemcpyAsync(ddesc.p, desc.data(), sizeof(BlockDesc) * nb, hipMemcpyHostToDevice, st));
-  hipLaunchKernelGGL(col_sign_batched_kernel, dim3((unsigned)ncol), dim3(256), 0, st,
-                     (const BlockDesc*)ddesc.p, (const long long*)dnoff.p, nb, (double*)dsign.p);
-  // V with its signs into J.V (or the other buffer, when J.V is the spare),
-  // W with the same order and signs into J.W (or the spare)
-  std::vector<PermJob> vj, wj;
+  // V and W in that order with V's signs into J.V and J.W, by way of the spare
+  // buffer where those hold the source
+  std::vector<PermJob> pj;
   std::vector<VecMove> moves;
   for (int b = 0; b < nb; ++b) {
     JacobiBlock& J = *blocks[b];
-    double* vdst = J.V == Vo[b] ? Vc[b] : J.V;
-    vj.push_back(PermJob{Vo[b], vdst, K[b], K[b], 0, noff[b]});
+    double* vdst = J.V == Vc[b] ? Vo[b] : J.V;
     double* wdst = J.W == Wc[b] ? Wo[b] : J.W;
-    wj.push_back(PermJob{Wc[b], wdst, L[b], K[b], 0, noff[b]});
+    pj.push_back(PermJob{Vc[b], vdst, K[b], K[b], 0, noff[b]});
+    pj.push_back(PermJob{Wc[b], wdst, L[b], K[b], 0, noff[b]});
     if (wdst != J.W) moves.push_back(VecMove{wdst, J.W, (long long)L[b] * K[b], kMoveF64, 0});
     if (vdst != J.V) moves.push_back(VecMove{vdst, J.V, (long long)K[b] * K[b], kMoveF64, 0});
   }
-  {
-    // the V moves read the identity permutation, the W moves the sort order
-    // (the second upload of the job table is queued behind the first launch)
-    std::swap(dperm.p, dident.p);
-    permute(vj, (const double*)dsign.p);
-    std::swap(dperm.p, dident.p);
-    permute(wj, (const double*)dsign.p);
-  }
-  if (!moves.empty()) {
-    long long mx = 0;
-    for (auto& m : moves) mx = std::max(mx, m.n);
-    DevMem dm(c, sizeof(VecMove) * moves.size());
-    SU2_HIP(hipMemcpyAsync(dm.p, moves.data(), sizeof(VecMove) * moves.size(),
-                           hipMemcpyHostToDevice, st));
-    dev_move_batch(c, (const VecMove*)dm.p, (int)moves.size(), mx);
-  }
+  prepare_permute(pj);
+  upload();
+  hipLaunchKernelGGL(col_sign_batched_kernel, dim3((unsigned)ncol), dim3(256), 0, st, ddesc,
+                     (const long long*)dnoff.p, nb, dperm, (double*)dsign.p);
+  permute((int)pj.size(), (const double*)dsign.p);
+  dev_moves(c, moves);
   // no wait: the outputs are used in stream order, and the host results (s)
   // are already on the host
   SU2_HIP(hipGetLastError());

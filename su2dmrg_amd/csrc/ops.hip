@@ -1,5 +1,7 @@
 #include "ops.hpp"
 
+#include <algorithm>
+
 #include "common.hpp"
 #include "context.hpp"
 
@@ -7,11 +9,18 @@ namespace su2 {
 
 namespace {
 
-__global__ void scale_columns_kernel(double* __restrict__ x, int m, int n,
-                                     const double* __restrict__ f) {
-  const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= (long long)m * n) return;
-  x[e] *= f[e / m];
+constexpr int kScalesPerLaunch = 80;
+struct ScaleArgs {
+  ScaledColumns j[kScalesPerLaunch];
+};
+
+// blockIdx.y the matrix, 1024 elements per workgroup
+__global__ __launch_bounds__(256) void scaled_columns_kernel(const ScaleArgs args) {
+  const ScaledColumns J = args.j[blockIdx.y];
+  const long long n = (long long)J.rows * J.cols;
+  const long long e0 = (long long)blockIdx.x * 1024;
+  for (long long e = e0 + threadIdx.x; e < min(e0 + 1024, n); e += 256)
+    J.dst[e] = J.src[e] * J.f[e / J.rows];
 }
 
 }  // namespace
@@ -44,19 +53,39 @@ void GemmBatch::run(Context& c, int variant) {
 
 void ScatterBatch::add(const void* key, const StridedAxpy& d) {
   if (d.rows <= 0 || d.cols <= 0) return;
-  int w = count_[key]++;
-  if ((int)waves_.size() <= w) waves_.resize(w + 1);
-  waves_[w].push_back(d);
+  auto it = last_.find(key);
+  int launch = 0;
+  if (it != last_.end()) {
+    StridedSum& g = launches_[it->second.first][it->second.second];
+    const StridedAxpy& h = g[0];
+    if (h.dst == d.dst && h.rs == d.rs && h.cs == d.cs && h.rows == d.rows && h.cols == d.cols &&
+        (h.src != nullptr) == (d.src != nullptr)) {
+      g.push_back(d);
+      return;
+    }
+    launch = it->second.first + 1;
+  }
+  if ((int)launches_.size() <= launch) launches_.resize(launch + 1);
+  launches_[launch].push_back(StridedSum{d});
+  last_[key] = {launch, (int)launches_[launch].size() - 1};
 }
 
-void ScatterBatch::run(Context& c) { dev_strided_axpy_launches(c, waves_); }
+void ScatterBatch::run(Context& c) { dev_strided_axpy_launches(c, launches_); }
 
-void dev_scale_columns(Context& c, double* x, int m, int n, const double* d_f) {
-  const long long tot = (long long)m * n;
-  if (tot <= 0) return;
-  hipLaunchKernelGGL(scale_columns_kernel, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0,
-                     c.stream(), x, m, n, d_f);
-  SU2_HIP(hipGetLastError());
+void dev_scaled_columns(Context& c, const std::vector<ScaledColumns>& jobs) {
+  ScaleArgs args;
+  for (size_t i0 = 0; i0 < jobs.size(); i0 += kScalesPerLaunch) {
+    const int n = (int)std::min<size_t>(kScalesPerLaunch, jobs.size() - i0);
+    long long most = 0;
+    for (int i = 0; i < n; ++i) {
+      args.j[i] = jobs[i0 + i];
+      most = std::max(most, (long long)args.j[i].rows * args.j[i].cols);
+    }
+    if (most <= 0) continue;
+    hipLaunchKernelGGL(scaled_columns_kernel, dim3((unsigned)((most + 1023) / 1024), n), dim3(256),
+                       0, c.stream(), args);
+    SU2_HIP(hipGetLastError());
+  }
 }
 
 }  // namespace su2

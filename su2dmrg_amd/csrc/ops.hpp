@@ -28,20 +28,28 @@ class GemmBatch {
   int n_ = 0;
 };
 
-// Strided scale-adds (StridedAxpy) collected with a destination key; entries
-// that hit the same key go to successive launches ("waves"), so every launch
-// writes disjoint elements and the sum order is the order of add().
+// Strided scale-adds (StridedAxpy) collected with a destination key.  Entries
+// of one key are summed in the order of add(): those that write the same
+// elements in the same layout one after the other in a thread, others in
+// successive launches.  Entries of different keys write disjoint elements.
 class ScatterBatch {
  public:
   void add(const void* key, const StridedAxpy& d);
   void run(Context& c);
 
  private:
-  std::map<const void*, int> count_;
-  std::vector<std::vector<StridedAxpy>> waves_;
+  std::map<const void*, std::pair<int, int>> last_;   // key -> launch and group of its last entry
+  std::vector<std::vector<StridedSum>> launches_;
 };
 
-// x[:, j] *= f[j] for the n columns of an m x n column-major matrix (ld m).
-void dev_scale_columns(Context& c, double* x, int m, int n, const double* d_f);
+// dst[:, j] = f[j] * src[:, j] for the cols columns of rows contiguous
+// elements each, many matrices in a launch (descriptors as kernel arguments).
+struct ScaledColumns {
+  double* dst;
+  const double* src;
+  const double* f;
+  int rows, cols;
+};
+void dev_scaled_columns(Context& c, const std::vector<ScaledColumns>& jobs);
 
 }  // namespace su2

@@ -398,7 +398,7 @@ __global__ __launch_bounds__(1024) void hh_apply_kernel(const PDesc* __restrict_
 
 // rk of every block: one past the last nonzero diagonal entry of Rc (a
 // dropped pivot leaves its whole row exactly zero)
-__global__ __launch_bounds__(256) void rank_prefix_kernel(const PDesc* __restrict__ desc,
+__global__ __launch_bounds__(256) void rank_prefix_kernel(PDesc* __restrict__ desc,
                                                           int* __restrict__ rk) {
   const PDesc D = desc[blockIdx.x];
   __shared__ int s[256];
@@ -411,7 +411,7 @@ __global__ __launch_bounds__(256) void rank_prefix_kernel(const PDesc* __restric
     if ((int)threadIdx.x < w) s[threadIdx.x] = max(s[threadIdx.x], s[threadIdx.x + w]);
     __syncthreads();
   }
-  if (threadIdx.x == 0) rk[blockIdx.x] = s[0] + 1;
+  if (threadIdx.x == 0) desc[blockIdx.x].rk = rk[blockIdx.x] = s[0] + 1;
 }
 
 __global__ void eye_batched_kernel(const PDesc* __restrict__ desc) {
@@ -481,13 +481,11 @@ void precondition_jacobi(Context& c, std::vector<PrecondBlock>& blocks) {
   // whose panels are identity reflectors and whose updates change nothing;
   // one wait brings the counts back to bound the panel loops
   {
-    DevBuf drk(c, (nb + 1) / 2);
-    hipLaunchKernelGGL(rank_prefix_kernel, dim3(nb), dim3(256), 0, st, dd, (int*)drk.p);
-    std::vector<int> rk(nb);
-    SU2_HIP(hipMemcpyAsync(rk.data(), drk.p, sizeof(int) * nb, hipMemcpyDeviceToHost, st));
+    int* rk = (int*)c.host_scratch((nb + 1) / 2);
+    hipLaunchKernelGGL(rank_prefix_kernel, dim3(nb), dim3(256), 0, st, (PDesc*)ddesc.p, rk);
+    SU2_HIP(hipGetLastError());
     SU2_HIP(hipStreamSynchronize(st));
     for (int i = 0; i < nb; ++i) hd[i].rk = rk[i];
-    SU2_HIP(hipMemcpyAsync(ddesc.p, hd.data(), sizeof(PDesc) * nb, hipMemcpyHostToDevice, st));
   }
   int rkmax = 0;
   for (int i = 0; i < nb; ++i) rkmax = std::max(rkmax, hd[i].rk);

@@ -48,8 +48,13 @@ struct SmallDesc {
   const double* A;
   double* W;
   double* V;
-  double* out;       // k squared singular values, then sweeps and worst squared overlap
+  double* out;       // k squared singular values, then sweeps and worst squared overlap (pinned)
   int m, n, ld;
+};
+
+constexpr int kBlocksPerLaunch = 64;   // descriptors travel as kernel arguments
+struct SmallArgs {
+  SmallDesc d[kBlocksPerLaunch];
 };
 
 // Lanes per pair (see above).
@@ -261,7 +266,7 @@ __device__ __forceinline__ int run_sweeps(double* X, double* nrm, const Shape& S
   return sweep;
 }
 
-__global__ __launch_bounds__(kThreads, 1) void small_svd_kernel(const SmallDesc* __restrict__ desc,
+__global__ __launch_bounds__(kThreads, 1) void small_svd_kernel(const SmallArgs args,
                                                                 double tol, double tol_abs,
                                                                 double noise_rel,
                                                                 int max_sweeps) {
@@ -271,7 +276,7 @@ __global__ __launch_bounds__(kThreads, 1) void small_svd_kernel(const SmallDesc*
   double* const s_p = s_inv;   // the pivot row of a reflector
   __shared__ int s_pos[kMaxK];
   __shared__ unsigned long long s_worst[2];
-  const SmallDesc D = desc[blockIdx.x];
+  const SmallDesc D = args.d[blockIdx.x];
   const int L = max(D.m, D.n), k = min(D.m, D.n), ld = D.ld;
   const int G = pair_lanes(k), NW = row_pairs(L, k), Lp = 2 * G * NW, rows = 2 * Lp;
   const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -493,24 +498,27 @@ int small_svd_batched(Context& c, const std::vector<JacobiBlock*>& blocks, doubl
     desc[i] = SmallDesc{b.A, b.W, b.V, nullptr, b.m, b.n, column_pitch(L, k)};
     lds = std::max(lds, sizeof(double) * (size_t)desc[i].ld * k);
   }
-  DevBuf out(c, tot);
-  for (int i = 0; i < nb; ++i) desc[i].out = out.p + off[i];
-  DevBuf dd(c, (long long)((sizeof(SmallDesc) * nb + 7) / 8));
-  SU2_HIP(hipMemcpyAsync(dd.p, desc.data(), sizeof(SmallDesc) * nb, hipMemcpyHostToDevice, st));
+  double* host = c.host_scratch(tot);
   SU2_HIP(hipFuncSetAttribute((const void*)small_svd_kernel,
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  hipLaunchKernelGGL(small_svd_kernel, dim3(nb), dim3(kThreads), lds, st,
-                     (const SmallDesc*)dd.p, tol, tol_abs, noise_rel, max_sweeps);
-  SU2_HIP(hipGetLastError());
-  std::vector<double> host(tot);
-  SU2_HIP(hipMemcpyAsync(host.data(), out.p, sizeof(double) * tot, hipMemcpyDeviceToHost, st));
+  for (int i0 = 0; i0 < nb; i0 += kBlocksPerLaunch) {
+    SmallArgs args;
+    const int n = std::min(kBlocksPerLaunch, nb - i0);
+    for (int i = 0; i < n; ++i) {
+      args.d[i] = desc[i0 + i];
+      args.d[i].out = host + off[i0 + i];
+    }
+    hipLaunchKernelGGL(small_svd_kernel, dim3(n), dim3(kThreads), lds, st, args, tol, tol_abs,
+                       noise_rel, max_sweeps);
+    SU2_HIP(hipGetLastError());
+  }
   SU2_HIP(hipStreamSynchronize(st));
   int sweeps = 0;
   double w = 0.0;
   for (int i = 0; i < nb; ++i) {
     JacobiBlock& b = *blocks[i];
     const int k = std::min(b.m, b.n);
-    const double* h = host.data() + off[i];
+    const double* h = host + off[i];
     b.s.resize(k);
     for (int j = 0; j < k; ++j) b.s[j] = std::sqrt(h[j]);
     sweeps = std::max(sweeps, (int)h[k]);

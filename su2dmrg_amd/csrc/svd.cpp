@@ -67,8 +67,11 @@ void svd_values(std::vector<Sec>& secs, std::vector<std::vector<double>>& wv, do
   }
 }
 
-// Global cut and output tensors of one wavefunction (columns already scaled).
-SvdResult svd_cut(Context& c, const Tensor& psi, std::vector<Sec>& secs, int max_dcut) {
+// Global cut and output tensors of one wavefunction; the kept columns times
+// their factors go to `outs`, which fill every element of both tensors.
+SvdResult svd_cut(Context& c, const Tensor& psi, std::vector<Sec>& secs, int max_dcut,
+                  const double* dfac, const std::vector<long long>& foff,
+                  std::vector<ScaledColumns>& outs) {
   std::vector<double> wsort;
   std::vector<int> isort;
   for (size_t i = 0; i < secs.size(); ++i) {
@@ -105,8 +108,8 @@ SvdResult svd_cut(Context& c, const Tensor& psi, std::vector<Sec>& secs, int max
   Leg la = psi.leg(0), lb = psi.leg(1);
   la.dir = 1;
   lb.dir = 1;
-  res.U.reset(new Tensor(&c, {la, res.bond}, 0, nullptr));
-  res.V.reset(new Tensor(&c, {lb, res.bond}, 0, nullptr));
+  res.U.reset(new Tensor(&c, {la, res.bond}, 0, nullptr, false));
+  res.V.reset(new Tensor(&c, {lb, res.bond}, 0, nullptr, false));
   for (size_t i = 0; i < secs.size(); ++i) {
     const Sec& s = secs[i];
     const int d = keep[i];
@@ -115,6 +118,9 @@ SvdResult svd_cut(Context& c, const Tensor& psi, std::vector<Sec>& secs, int max
     // kept columns are the last d of the k (ascending singular values)
     const double* Ucols;
     const double* Vcols;
+    // factors of the long side (held in U), then of the short side
+    const double* fl = dfac + foff[i] + (k - d);
+    const double* fs = fl + k;
     if (s.m >= s.n) {
       Ucols = s.U.p + (long long)(k - d) * s.m;
       Vcols = s.V.p + (long long)(k - d) * k;
@@ -124,8 +130,11 @@ SvdResult svd_cut(Context& c, const Tensor& psi, std::vector<Sec>& secs, int max
     }
     const int bu = res.U->find2(s.twoj, s.twoj), bv = res.V->find2(s.twoj, s.twoj);
     SU2_CHECK(bu >= 0 && bv >= 0, kErrStructure, "svd: missing output block");
-    dev_copy(c, res.U->data() + res.U->blocks()[bu].offset, Ucols, (long long)s.m * d);
-    dev_copy(c, res.V->data() + res.V->blocks()[bv].offset, Vcols, (long long)s.n * d);
+    const bool tall = s.m >= s.n;
+    outs.push_back(ScaledColumns{res.U->data() + res.U->blocks()[bu].offset, Ucols, tall ? fl : fs,
+                                 s.m, d});
+    outs.push_back(ScaledColumns{res.V->data() + res.V->blocks()[bv].offset, Vcols, tall ? fs : fl,
+                                 s.n, d});
     std::vector<double> kv(s.s.begin() + (k - d), s.s.end());
     res.kept.push_back(kv);
   }
@@ -209,7 +218,7 @@ std::vector<SvdResult> truncated_svd_batch(Context& c, const std::vector<SvdJob>
       }
   }
   // column factors of every sector of every wavefunction: one upload, the
-  // scalings queued, no wait until the outputs are in place
+  // scaled copies queued, no wait until the outputs are in place
   std::vector<double> fac;
   std::vector<std::vector<long long>> foff(jobs.size());
   for (size_t q = 0; q < jobs.size(); ++q)
@@ -218,21 +227,15 @@ std::vector<SvdResult> truncated_svd_batch(Context& c, const std::vector<SvdJob>
   if (!fac.empty())
     SU2_HIP(hipMemcpyAsync(dfac.p, fac.data(), fac.size() * sizeof(double), hipMemcpyHostToDevice,
                            c.stream()));
-  for (size_t q = 0; q < jobs.size(); ++q)
-    for (size_t i = 0; i < secs[q].size(); ++i) {
-      Sec& s = secs[q][i];
-      if (s.k == 0) continue;
-      const int longrows = s.m >= s.n ? s.m : s.n;
-      dev_scale_columns(c, s.U.p, longrows, s.k, dfac.p + foff[q][i]);
-      dev_scale_columns(c, s.V.p, s.k, s.k, dfac.p + foff[q][i] + s.k);
-    }
+  std::vector<ScaledColumns> outs;
   std::vector<SvdResult> out;
   for (size_t q = 0; q < jobs.size(); ++q) {
-    out.push_back(svd_cut(c, *jobs[q].psi, secs[q], jobs[q].max_dcut));
+    out.push_back(svd_cut(c, *jobs[q].psi, secs[q], jobs[q].max_dcut, dfac.p, foff[q], outs));
     out.back().jacobi_sweeps = jacobi_sweeps;
     out.back().t_jacobi = t_jacobi / jobs.size();
     out.back().jacobi_worst = jacobi_worst;
   }
+  dev_scaled_columns(c, outs);
   SU2_HIP(hipStreamSynchronize(c.stream()));
   return out;
 }

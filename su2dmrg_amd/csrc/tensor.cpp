@@ -272,26 +272,9 @@ void ZeroBatch::add(Tensor& t) {
 }
 
 void ZeroBatch::run(Context& c) {
-  if (z_.empty()) return;
-  std::vector<VecMove> h(z_.size());
-  long long mx = 0;
-  for (size_t i = 0; i < z_.size(); ++i) {
-    h[i] = VecMove{nullptr, z_[i].first, z_[i].second, kZeroF64, 0};
-    mx = std::max(mx, z_[i].second);
-  }
-  // the descriptor block returns to the cache at once; stream order keeps it
-  // until the launch has read it
-  VecMove* d = (VecMove*)c.dev_alloc(h.size() * sizeof(VecMove));
-  try {
-    SU2_HIP(hipMemcpyAsync(d, h.data(), h.size() * sizeof(VecMove), hipMemcpyHostToDevice,
-                           c.stream()));
-    for (size_t i = 0; i < h.size(); i += 65535)
-      dev_move_batch(c, d + i, (int)std::min<size_t>(65535, h.size() - i), mx);
-  } catch (...) {
-    c.dev_free(d);
-    throw;
-  }
-  c.dev_free(d);
+  std::vector<VecMove> h;
+  for (auto& z : z_) h.push_back(VecMove{nullptr, z.first, z.second, kZeroF64, 0});
+  dev_moves(c, h);
   z_.clear();
 }
 
