@@ -1351,7 +1351,7 @@ static int jacobi_svd_large(Context& c, const std::vector<JacobiBlock*>& blocks,
       sort_permute(nullptr);
       for (int b : pre)
         pb.push_back(PrecondBlock{Wc[b], Vc[b], Wo[b], Vo[b], L[b], K[b], K[b], desc[b].normF, 0.0});
-      precondition_jacobi(c, pb);
+      precondition_jacobi(c, pb, plain);
       for (int b : pre) {
         std::swap(Wc[b], Wo[b]);
         std::swap(Vc[b], Vo[b]);
@@ -1386,7 +1386,7 @@ static int jacobi_svd_large(Context& c, const std::vector<JacobiBlock*>& blocks,
         back.push_back(VecMove{Vo[b] + vo, Vc[b] + vo, (long long)n * K[b], kMoveF64, 0});
       }
       if (!tail.empty()) {
-        precondition_jacobi(c, tail);
+        precondition_jacobi(c, tail, false);
         dev_moves(c, back);
       }
       if (!tail.empty()) norms();

@@ -147,7 +147,181 @@ __global__ __launch_bounds__(256) void chol_trail_kernel(const PDesc* __restrict
   }
 }
 
-// Householder QR of one 16-column panel of X (rows c0..K-1; row c0 + r on
+// Lane `src`'s x on every lane, in scalar registers.
+__device__ __forceinline__ double lane_value(double x, int src) {
+  union { double d; int i[2]; } u, v;
+  u.d = x;
+  v.i[0] = __builtin_amdgcn_readlane(u.i[0], src);
+  v.i[1] = __builtin_amdgcn_readlane(u.i[1], src);
+  return v.d;
+}
+
+// Orthogonal factor of one 16-column panel of X (rows c0..K-1) in compact WY
+// form, I - V T V^T = H_0 ... H_{b-1}.  A reflector needs inner products of the
+// updated columns; the panel's Gram matrix X^T X does not change under the
+// reflectors, so with it and the panel's first 16 rows one wave finds all 16 of
+// them without another pass: the products over the rows below row j are
+// (X^T X)_jc minus those over rows 0..j.  The same updates applied to an
+// identity give M with V = X M below the first 16 rows.  The differences lose
+// digits where a column nearly depends on those before it, so V need not
+// annihilate exactly; T^-1 = striu(V^T V) + diag(V^T V) / 2, taken from the V
+// that was stored, makes I - V T V^T orthogonal for any V, and only that counts
+// for a preconditioner.  A column whose remainder is below kDepends of it gets
+// no reflector.
+//
+// Three short phases on one workgroup, bound by the 16 dependent reflectors
+// (about 5 us) and, from about 1000 rows, by the 12 MFMAs per 16 rows on the
+// CU's four matrix cores.  Reducing every reflector's 16 products over the
+// workgroup took 65 us a panel against 21 in the sectors of a D = 2000 bond (up to 1383), 51 against
+// 14 on those of a 6x4 run up to d = 924.
+constexpr double kDepends = 1e-13;
+
+__global__ __launch_bounds__(PT) void wy_panel_kernel(const PDesc* __restrict__ desc, int p) {
+  const PDesc D = desc[blockIdx.x];
+  const int K = D.K, c0 = PB * p;
+  // a panel of zero columns (past the last nonzero pivot) is the identity
+  if (c0 >= D.rk) return;
+  const int bp = min(PB, K - c0), m = K - c0;
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  constexpr int NW = PT / 64;
+  const int row4 = lane >> 4, col = lane & 15;
+  __shared__ double s_part[NW][PB * PB];
+  __shared__ double s_g[PB][PB + 1], s_m[PB][PB + 1], s_v[PB][PB + 1];
+  static_assert(PB == 16, "16 x 16 x 4 MFMAs");
+  double* const X = D.G + (size_t)c0 * K + c0;   // row r, column c at X[r K + c]
+
+  // sum of the waves' 16 x 16 results (register r of lane l: row l/16 + 4 r, column l%16)
+  auto gather = [&](const f64x4& acc) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) s_part[wave][(row4 + 4 * r) * PB + col] = acc[r];
+    __syncthreads();
+    if (t < PB * PB) {
+      double v = 0.0;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) v += s_part[w][t];
+      s_g[t / PB][t % PB] = v;
+    }
+    __syncthreads();
+  };
+
+  // X^T X: four rows a step, the same register as both operands
+  {
+    f64x4 acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
+    for (int r0 = 4 * wave; r0 < m; r0 += 4 * NW) {
+      const int r = r0 + row4;
+      const double x = (r < m && col < bp) ? X[(size_t)r * K + col] : 0.0;
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(x, x, acc, 0, 0, 0);
+    }
+    gather(acc);
+  }
+
+  // the reflectors: lane c (of each 16) holds column c of the first 16 rows,
+  // of the Gram matrix and of M
+  unsigned used = 0;
+  if (wave == 0) {
+    double x[PB], g[PB], mm[PB];
+#pragma unroll
+    for (int r = 0; r < PB; ++r) {
+      x[r] = (r < m && col < bp) ? X[(size_t)r * K + col] : 0.0;
+      g[r] = s_g[r][col];
+      mm[r] = (r == col && col < bp) ? 1.0 : 0.0;
+    }
+    static_for<0, PB>([&](auto jc) {
+      constexpr int j = decltype(jc)::value;
+      if (j < bp) {
+        // products over the rows below j
+        double d = g[j];
+#pragma unroll
+        for (int r = 0; r <= j; ++r) d = fma(-lane_value(x[r], j), x[r], d);
+        const double alpha = lane_value(x[j], j), sig2 = lane_value(d, j),
+                     gjj = lane_value(g[j], j);
+        double tau = 0.0, scale = 0.0;
+        if (sig2 > kDepends * gjj) {
+          const double beta = -copysign(sqrt(fma(alpha, alpha, sig2)), alpha);
+          tau = (beta - alpha) / beta;
+          scale = 1.0 / (alpha - beta);
+          used |= 1u << j;
+        }
+        const double f = col > j ? -tau * fma(scale, d, x[j]) : 0.0;
+        if (col > j) x[j] += f;
+#pragma unroll
+        for (int r = j + 1; r < PB; ++r) {
+          const double v = lane_value(x[r], j) * scale;
+          x[r] = col == j ? v : fma(f, v, x[r]);
+        }
+#pragma unroll
+        for (int r = 0; r <= j; ++r) {
+          const double v = lane_value(mm[r], j) * scale;
+          mm[r] = col == j ? v : fma(f, v, mm[r]);
+        }
+      }
+    });
+    if (lane < PB) {
+#pragma unroll
+      for (int r = 0; r < PB; ++r) {
+        if (r < m && col < bp) X[(size_t)r * K + col] = x[r];
+        s_v[r][col] = (col >= bp || r < col) ? 0.0 : r == col ? 1.0 : x[r];
+        s_m[r][col] = mm[r];
+      }
+    }
+  }
+  __syncthreads();
+
+  // V = X M below them, 16 rows a step, and V^T V
+  {
+    f64x4 acc = {0.0, 0.0, 0.0, 0.0};
+    double b[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) b[s] = s_m[4 * s + row4][col];
+    if (wave == 0) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const double v = s_v[row4 + 4 * r][col];
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(v, v, acc, 0, 0, 0);
+      }
+    }
+#pragma unroll 2
+    for (int r0 = PB + PB * wave; r0 < m; r0 += PB * NW) {
+      double a[4];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const int r = r0 + col, c = 4 * s + row4;
+        a[s] = (r < m && c < bp) ? X[(size_t)r * K + c] : 0.0;
+      }
+      f64x4 y = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int s = 0; s < 4; ++s) y = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s], b[s], y, 0, 0, 0);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = r0 + row4 + 4 * r;
+        if (row < m && col < bp) X[(size_t)row * K + col] = y[r];
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(y[r], y[r], acc, 0, 0, 0);
+      }
+    }
+    gather(acc);
+  }
+
+  // T by back substitution, column c on lane c
+  if (wave == 0) {
+    const double inv = (used >> col & 1u) ? 2.0 / s_g[col][col] : 0.0;
+    double tc[PB];
+    static_for<0, PB>([&](auto ic) {
+      constexpr int i = PB - 1 - decltype(ic)::value;
+      double acc = i == col ? 1.0 : 0.0;
+#pragma unroll
+      for (int k = i + 1; k < PB; ++k) acc = fma(-s_g[i][k], tc[k], acc);
+      tc[i] = acc * lane_value(inv, i);
+    });
+    if (lane < PB)
+#pragma unroll
+      for (int i = 0; i < PB; ++i) D.T[(size_t)p * PB * PB + i + PB * col] = tc[i];
+  }
+}
+
+// Householder QR of one 16-column panel of X for the plain iteration, which
+// keeps every direction down to rounding and its bits (rows c0..K-1; row c0 + r on
 // thread r % 1024, in registers).
 // Column j becomes its Householder vector below the diagonal (the unit
 // diagonal implicit); the panel's T factor of the compact WY form H_0 ...
@@ -425,7 +599,7 @@ unsigned cdiv(long long a, long long b) { return (unsigned)((a + b - 1) / b); }
 
 }  // namespace
 
-void precondition_jacobi(Context& c, std::vector<PrecondBlock>& blocks) {
+void precondition_jacobi(Context& c, std::vector<PrecondBlock>& blocks, bool plain) {
   const int nb = (int)blocks.size();
   if (nb == 0) return;
   SU2_CHECK(nb < 65536, kErrCapacity, "jacobi preconditioner: %d blocks", nb);
@@ -492,7 +666,7 @@ void precondition_jacobi(Context& c, std::vector<PrecondBlock>& blocks) {
   const int npq = (rkmax + PB - 1) / PB;
   // Householder QR of Rc^T by column panels (trailing columns updated)
   for (int p = 0; p < npq; ++p) {
-    hipLaunchKernelGGL(hh_panel_kernel, dim3(nb), dim3(PT), 0, st, dd, p);
+    hipLaunchKernelGGL(plain ? hh_panel_kernel : wy_panel_kernel, dim3(nb), dim3(PT), 0, st, dd, p);
     const int n = rkmax - PB * (p + 1);
     if (n > 0) {
       hipLaunchKernelGGL(hh_apply_kernel, dim3(cdiv(n, PB), nb), dim3(1024), 0, st, dd, p, 1);
