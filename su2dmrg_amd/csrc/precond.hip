@@ -43,74 +43,82 @@ __device__ __forceinline__ void static_for(F&& f) {
   }
 }
 
-// Upper Cholesky of G by one 16-row panel: rows c0..c0+bp-1, columns
-// c0..K-1, column j of the row panel on thread j % 1024, in registers.  A
-// pivot at or below tiny (or
-// negative from rounding) gives a zero row.  One barrier per step: row k is
-// published before its pivot is used, into alternating LDS buffers.
-__global__ __launch_bounds__(PT) void chol_panel_kernel(const PDesc* __restrict__ desc, int p) {
-  const PDesc D = desc[blockIdx.x];
+// Lane `src`'s x on every lane, in scalar registers.
+__device__ __forceinline__ double lane_value(double x, int src) {
+  union { double d; int i[2]; } u, v;
+  u.d = x;
+  v.i[0] = __builtin_amdgcn_readlane(u.i[0], src);
+  v.i[1] = __builtin_amdgcn_readlane(u.i[1], src);
+  return v.d;
+}
+
+// Upper Cholesky of G by one 16-row panel: rows c0..c0+bp-1, columns c0..K-1.
+// A pivot at or below tiny (or negative from rounding) gives a zero row.
+// Bound by the 16 dependent pivots: every workgroup factors the 16 x 16
+// diagonal block for itself in one wave, column c on lane c, without barriers,
+// and then solves 256 further columns, one per thread.  The factor of the
+// diagonal block goes to D.T (workgroups still read the block);
+// rank_prefix_kernel puts it in place.  One workgroup for all columns with a
+// barrier per pivot took 27 us a panel in the sectors of a D = 2000 bond where
+// this takes 12, 16 against 8 on a 6x4 run's blocks.
+constexpr int kCholCols = 256;
+
+__global__ __launch_bounds__(kCholCols) void chol_panel_kernel(const PDesc* __restrict__ desc,
+                                                               int p) {
+  const PDesc D = desc[blockIdx.y];
   const int K = D.K, c0 = PB * p;
   if (c0 >= K) return;
   const int bp = min(PB, K - c0), nc = K - c0;
-  const int t = threadIdx.x;
-  __shared__ double s_raw[2][PB];
-  double w[PROWS][PB];
-  double* gcol[PROWS];
+  const int j0 = PB + (int)blockIdx.x * kCholCols;
+  if (blockIdx.x > 0 && j0 >= nc) return;
+  const int t = threadIdx.x, j = j0 + t;
+  // -R[k][i] / R[k][k]-scaled multipliers and the inverse pivots
+  __shared__ double s_f[PB][PB], s_inv[PB];
+  double w[PB];
+  double* const gcol = D.G + (size_t)(c0 + min(j, nc - 1)) * K + c0;
 #pragma unroll
-  for (int q = 0; q < PROWS; ++q) {
-    const int j = t + PT * q;
-    gcol[q] = D.G + (size_t)(c0 + min(j, nc - 1)) * K + c0;
-  }
-#pragma unroll
-  for (int q = 0; q < 2; ++q) {
-    const int j = t + PT * q;
-#pragma unroll
-    for (int i = 0; i < PB; ++i) w[q][i] = (j < nc && i < bp) ? gcol[q][i] : 0.0;
-  }
-  static_for<0, PB>([&](auto kc) {
-    constexpr int k = decltype(kc)::value;
-    __builtin_amdgcn_sched_barrier(0);
-    if (k < bp) {
-      double* raw = s_raw[k & 1];
-      // row k as it stands (columns c0 + k .. c0 + 15 live on threads k..15)
-      if (t >= k && t < PB) raw[t] = w[0][k];
-      __syncthreads();
-      const double dk = raw[k];
-      const double inv = dk > D.tiny ? 1.0 / sqrt(dk) : 0.0;
-      // R[k][j] for my columns (zero left of the diagonal), then the rows
-      // below: w[i][j] -= R[k][i] R[k][j] for k < i <= j (row by row, so
-      // that each R[k][i] is live for one row only)
-      double rkj[PROWS];
-#pragma unroll
-      for (int q = 0; q < PROWS; ++q) {
-        const int j = t + PT * q;
-        rkj[q] = (j >= k) ? w[q][k] * inv : 0.0;
-        w[q][k] = rkj[q];
-      }
-#pragma unroll
-      for (int i = k + 1; i < PB; ++i) {
-        if (i >= bp) continue;
-        const double f = -raw[i] * inv;
-#pragma unroll
-        for (int q = 0; q < PROWS; ++q)
-          if (i <= t + PT * q) w[q][i] = fma(f, rkj[q], w[q][i]);
-      }
-    }
-  });
-#pragma unroll
-  for (int q = 0; q < 2; ++q) {
-    const int j = t + PT * q;
-    if (j >= nc) continue;
+  for (int i = 0; i < PB; ++i) w[i] = (j < nc && i < bp) ? gcol[i] : 0.0;
+  if (t < 64) {
+    const int c = t & 15;
+    double d[PB];
 #pragma unroll
     for (int i = 0; i < PB; ++i)
-      if (i < bp) gcol[q][i] = (i > j) ? 0.0 : w[q][i];
+      d[i] = (c < bp && i < bp) ? D.G[(size_t)(c0 + c) * K + c0 + i] : 0.0;
+    static_for<0, PB>([&](auto kc) {
+      constexpr int k = decltype(kc)::value;
+      const double dk = lane_value(d[k], k);
+      const double inv = (k < bp && dk > D.tiny) ? 1.0 / sqrt(dk) : 0.0;
+      const double rk = c >= k ? d[k] * inv : 0.0;
+      // lane i's f multiplies row k into row i
+      const double fi = -d[k] * inv;
+      if (t < PB) s_f[k][t] = fi;
+      if (t == 0) s_inv[k] = inv;
+#pragma unroll
+      for (int i = k + 1; i < PB; ++i) {
+        const double f = lane_value(fi, i);
+        if (i <= c) d[i] = fma(f, rk, d[i]);
+      }
+      d[k] = rk;
+    });
+    if (blockIdx.x == 0 && t < PB)
+#pragma unroll
+      for (int i = 0; i < PB; ++i)
+        D.T[(size_t)p * PB * PB + i + PB * t] = i <= t ? d[i] : 0.0;
   }
-  // the panel's columns below its diagonal block: zero (Rc is upper
-  // triangular, and read row-major they are X's entries above its diagonal)
-  for (int e = t; e < bp * (nc - bp); e += PT) {
-    const int i = e / (nc - bp), r = e % (nc - bp);
-    D.G[(size_t)(c0 + bp + r) + (size_t)(c0 + i) * K] = 0.0;
+  __syncthreads();
+  if (j < nc) {
+    static_for<0, PB>([&](auto kc) {
+      constexpr int k = decltype(kc)::value;
+      w[k] *= s_inv[k];
+#pragma unroll
+      for (int i = k + 1; i < PB; ++i) w[i] = fma(s_f[k][i], w[k], w[i]);
+    });
+#pragma unroll
+    for (int i = 0; i < PB; ++i)
+      if (i < bp) gcol[i] = w[i];
+    // the panel's columns below its diagonal block: zero (Rc is upper
+    // triangular, and read row-major they are X's entries above its diagonal)
+    for (int i = 0; i < bp; ++i) D.G[(size_t)(c0 + j) + (size_t)(c0 + i) * K] = 0.0;
   }
 }
 
@@ -145,15 +153,6 @@ __global__ __launch_bounds__(256) void chol_trail_kernel(const PDesc* __restrict
       D.G[(size_t)gi + (size_t)gj * K] -= acc;
     }
   }
-}
-
-// Lane `src`'s x on every lane, in scalar registers.
-__device__ __forceinline__ double lane_value(double x, int src) {
-  union { double d; int i[2]; } u, v;
-  u.d = x;
-  v.i[0] = __builtin_amdgcn_readlane(u.i[0], src);
-  v.i[1] = __builtin_amdgcn_readlane(u.i[1], src);
-  return v.d;
 }
 
 // Orthogonal factor of one 16-column panel of X (rows c0..K-1) in compact WY
@@ -452,22 +451,17 @@ __global__ __launch_bounds__(PT) void hh_panel_kernel(const PDesc* __restrict__ 
   if (t < PB * PB) D.T[(size_t)p * PB * PB + t] = s_T[t % PB][t / PB];
 }
 
-// Householder vector i of panel p at panel row r (the unit diagonal implicit).
-__device__ __forceinline__ double hh_v(const PDesc& D, int c0, int bp, int m, int i, int r) {
-  if (i >= bp || r >= m || r < i) return 0.0;
-  if (r == i) return 1.0;
-  return D.G[(size_t)(c0 + r) * D.K + (c0 + i)];
-}
-
 // A <- A - V op(T) (V^T A) for 16 columns of A (rows c0..K-1): A = X from
 // column c0 + bp (the QR's trailing columns, op(T) = T^T) or A = Q from
 // column c0 (Q2's backward formation, op(T) = T).  One workgroup owns its 16
 // columns over every row, so the products and the update need no other
-// workgroup.  1024 threads: 256-row chunks of V and A staged through LDS,
-// each of the 16 waves accumulating V^T A over its 16 rows of every chunk
-// on the matrix cores (four 16x16x4 FP64 MFMAs), the 16 partial products
-// summed in wave order, Z = op(T) sums in LDS; then A -= V Z by the same
-// waves, a 16 x 16 tile each on the matrix cores.
+// workgroup.  Each of the 16 waves takes every 16th tile of 16 rows: its tiles
+// of A stay in registers between the two products (an accumulator's layout is
+// that of a B operand), V comes from memory in the layout of either product,
+// and the only exchange is the sum of the waves' V^T A in wave order.  Bound
+// by the latency of its loads; staging V and A through LDS in 256-row chunks,
+// two barriers each, took 27 us in the sectors of a D = 2000 bond where this
+// takes 17, 8.6 against 6 on a 6x4 run's blocks.
 __global__ __launch_bounds__(1024) void hh_apply_kernel(const PDesc* __restrict__ desc, int p,
                                                         int qr) {
   const PDesc D = desc[blockIdx.y];
@@ -479,62 +473,50 @@ __global__ __launch_bounds__(1024) void hh_apply_kernel(const PDesc* __restrict_
   const int chunk = blockIdx.x * PB;
   if (chunk >= ncols) return;
   // A(row, col): X row-major (the QR's trailing columns) or Q column-major
-  double* A = qr ? D.G : D.Q;
   const size_t rs = qr ? (size_t)K : 1, cs = qr ? 1 : (size_t)K;
-  constexpr int NG = 4;
-  __shared__ double sv[NG][64][PB + 1], sa[NG][64][PB + 1];
-  __shared__ double sp[16][PB][PB + 1];   // the waves' partial V^T A
+  double* const A = (qr ? D.G : D.Q) + (size_t)c0 * rs + (size_t)(colstart + chunk) * cs;
+  const double* const X = D.G + (size_t)c0 * K + c0;   // row r, column c at X[r K + c]
+  constexpr int NW = 16, TILES = kPrecondMaxK / (PB * NW);
+  __shared__ double sp[NW][PB][PB + 1];   // the waves' partial V^T A
   __shared__ double sz[PB][PB + 1];
-  static_assert(PB == 16 && NG * 4 == 16, "16 waves of 16 rows per 256-row chunk");
-  const int t = threadIdx.x, g = t / 256, tg = t % 256;
-  const int i = tg / PB, c = tg % PB;
-  const int lane = t & 63, wave = t >> 6, gw = wave >> 2, rw = (wave & 3) * 16;
+  static_assert(PB == 16 && TILES * PB * NW == kPrecondMaxK, "16 waves of 16-row tiles");
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int row4 = lane >> 4, col = lane & 15;
+  const bool mine = chunk + col < ncols;
+  // Householder vector i at panel row r (the unit diagonal implicit)
+  auto hh_v = [&](int i, int r) {
+    const double v = (i < bp && r < m) ? X[(size_t)r * K + i] : 0.0;
+    return i >= bp || r < i ? 0.0 : r == i ? 1.0 : v;
+  };
+  double a[TILES][4];
   f64x4 pacc = {0.0, 0.0, 0.0, 0.0};
-  // every thread runs the same iterations (the barriers inside need that);
-  // a group past the last row loads zeros
-  for (int base = 0; base < m; base += 64 * NG) {
-    const int r0 = base + 64 * g;
-    for (int e = tg; e < 64 * PB; e += 256) {
-      // X: the 16 columns of a row are contiguous, so k runs fastest
-      const int rr = e / PB, k = e % PB;
-      const int r = r0 + rr;
-      sv[g][rr][k] = hh_v(D, c0, bp, m, k, r);
-      if (qr) {
-        const int col = chunk + k;
-        sa[g][rr][k] = (r < m && col < ncols) ? A[(size_t)(c0 + r) * rs + (size_t)(colstart + col) * cs] : 0.0;
-      }
-    }
-    if (!qr) {
-      for (int e = tg; e < 64 * PB; e += 256) {
-        // Q: the rows of a column are contiguous, so rr runs fastest
-        const int rr = e % 64, k = e / 64;
-        const int r = r0 + rr, col = chunk + k;
-        sa[g][rr][k] = (r < m && col < ncols) ? A[(size_t)(c0 + r) * rs + (size_t)(colstart + col) * cs] : 0.0;
-      }
-    }
-    __syncthreads();
-    // (V^T A)[a][b] += sum over 4 rows: lane l feeds V[row l/16][l%16] as
+#pragma unroll
+  for (int q = 0; q < TILES; ++q) {
+    const int r0 = (q * NW + wave) * PB;
+    if (r0 >= m) continue;
+    // (V^T A)[i][c] += sum over 4 rows: lane l feeds V[row l/16][l%16] as
     // the A operand and A[row l/16][l%16] as the B operand
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int rr = rw + 4 * j + (lane >> 4);
-      pacc = __builtin_amdgcn_mfma_f64_16x16x4f64(sv[gw][rr][lane & 15], sa[gw][rr][lane & 15],
-                                                  pacc, 0, 0, 0);
+    for (int s = 0; s < 4; ++s) {
+      const int r = r0 + 4 * s + row4;
+      a[q][s] = (r < m && mine) ? A[(size_t)r * rs + (size_t)col * cs] : 0.0;
+      pacc = __builtin_amdgcn_mfma_f64_16x16x4f64(hh_v(col, r), a[q][s], pacc, 0, 0, 0);
     }
-    __syncthreads();
   }
   // result register r of lane l is row l/16 + 4 r, column l % 16
 #pragma unroll
-  for (int r = 0; r < 4; ++r) sp[wave][(lane >> 4) + 4 * r][lane & 15] = pacc[r];
+  for (int r = 0; r < 4; ++r) sp[wave][row4 + 4 * r][col] = pacc[r];
   __syncthreads();
-  if (g == 0) {
+  const int i = t / PB, c = t % PB;
+  if (t < PB * PB) {
     double v = 0.0;
 #pragma unroll
-    for (int w = 0; w < 16; ++w) v += sp[w][i][c];
+    for (int w = 0; w < NW; ++w) v += sp[w][i][c];
     sp[0][i][c] = v;   // row i of wave 0's block is read by this thread only
   }
   __syncthreads();
-  if (g == 0) {
+  if (t < PB * PB) {
     const double* T = D.T + (size_t)p * PB * PB;   // T[a][b] at a + 16 b
     double z = 0.0;
 #pragma unroll
@@ -542,43 +524,40 @@ __global__ __launch_bounds__(1024) void hh_apply_kernel(const PDesc* __restrict_
     sz[i][c] = (chunk + c < ncols) ? z : 0.0;
   }
   __syncthreads();
-  // A -= V Z: each wave a 16 x 16 tile of the 256-row chunk on the matrix
-  // cores (lane l feeds V[row l%16][k] and Z[k][l%16], k = 4 j + l/16), the
-  // result subtracted from A (lane l: rows l/16 + 4 r, column l % 16)
-  for (int base = 0; base < m; base += 64 * NG) {
-    const int r0 = base + 64 * g;
-    for (int e = tg; e < 64 * PB; e += 256) {
-      const int rr = e / PB, k = e % PB;
-      sv[g][rr][k] = hh_v(D, c0, bp, m, k, r0 + rr);
-    }
-    __syncthreads();
+  // A -= V Z: lane l feeds V[row l%16][k] and Z[k][l%16], k = 4 s + l/16
+#pragma unroll
+  for (int q = 0; q < TILES; ++q) {
+    const int r0 = (q * NW + wave) * PB;
+    if (r0 >= m) continue;
     f64x4 y = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int k = 4 * j + (lane >> 4);
-      y = __builtin_amdgcn_mfma_f64_16x16x4f64(sv[gw][rw + (lane & 15)][k], sz[k][lane & 15], y,
-                                               0, 0, 0);
+    for (int s = 0; s < 4; ++s) {
+      const int k = 4 * s + row4;
+      y = __builtin_amdgcn_mfma_f64_16x16x4f64(hh_v(k, r0 + col), sz[k][col], y, 0, 0, 0);
     }
-    const int cc = lane & 15;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int row = base + 64 * gw + rw + (lane >> 4) + 4 * r;
-      if (row < m && chunk + cc < ncols)
-        A[(size_t)(c0 + row) * rs + (size_t)(colstart + chunk + cc) * cs] -= y[r];
+      const int row = r0 + row4 + 4 * r;
+      if (row < m && mine) A[(size_t)row * rs + (size_t)col * cs] = a[q][r] - y[r];
     }
-    __syncthreads();
   }
 }
 
-// rk of every block: one past the last nonzero diagonal entry of Rc (a
-// dropped pivot leaves its whole row exactly zero)
+// The Cholesky's diagonal blocks into place, and rk of every block: one past
+// the last nonzero diagonal entry of Rc (a dropped pivot leaves its whole row
+// exactly zero).
 __global__ __launch_bounds__(256) void rank_prefix_kernel(PDesc* __restrict__ desc,
                                                           int* __restrict__ rk) {
   const PDesc D = desc[blockIdx.x];
   __shared__ int s[256];
   int last = -1;
-  for (int i = threadIdx.x; i < D.K; i += 256)
-    if (D.G[(size_t)i + (size_t)i * D.K] != 0.0) last = max(last, i);
+  const int i = threadIdx.x % PB, j = threadIdx.x / PB;
+  for (int c0 = 0; c0 < D.K; c0 += PB) {
+    if (c0 + i >= D.K || c0 + j >= D.K) continue;
+    const double v = D.T[(size_t)c0 * PB + i + PB * j];
+    D.G[(size_t)(c0 + i) + (size_t)(c0 + j) * D.K] = v;
+    if (i == j && v != 0.0) last = max(last, c0 + i);
+  }
   s[threadIdx.x] = last;
   __syncthreads();
   for (int w = 128; w > 0; w >>= 1) {
@@ -643,8 +622,9 @@ void precondition_jacobi(Context& c, std::vector<PrecondBlock>& blocks, bool pla
   const int npmax = (kmax + PB - 1) / PB;
   // Cholesky by row panels
   for (int p = 0; p < npmax; ++p) {
-    hipLaunchKernelGGL(chol_panel_kernel, dim3(nb), dim3(PT), 0, st, dd, p);
     const int n = kmax - PB * (p + 1);
+    hipLaunchKernelGGL(chol_panel_kernel, dim3(std::max(1u, cdiv(std::max(n, 0), kCholCols)), nb),
+                       dim3(kCholCols), 0, st, dd, p);
     if (n > 0) {
       const unsigned nt = cdiv(n, 64);
       hipLaunchKernelGGL(chol_trail_kernel, dim3(nt, nt, nb), dim3(256), 0, st, dd, p);
