@@ -31,13 +31,6 @@ constexpr double kNoiseRel = 1e-13;
 // Blocks under this many columns are preconditioned whatever the setting says:
 // a 192 x 192 block takes 5.5 ms that way and 14.4 ms without.
 constexpr int kPrecondAlways = 256;
-// Columns a first preconditioning pass left at or below this part of ||A||_F
-// (the square root of the pivot floor) are preconditioned again, if there are
-// at least kTailMin of them; there, pivots at or below kTailNoise ||A||_F are
-// the rounding of the first pass.
-constexpr double kTailRel = 3.2e-8;
-constexpr int kTailMin = 32;
-constexpr double kTailNoise = 3e-14;
 constexpr double kTolAbs = 1e-14;   // rounding floor of a pair, relative to ||A||_F
 
 typedef double f64x4 __attribute__((ext_vector_type(4)));
@@ -1334,7 +1327,13 @@ static int jacobi_svd_large(Context& c, const std::vector<JacobiBlock*>& blocks,
     upload();
     permute((int)pj.size(), nullptr);
   };
-  // QR preconditioning (precond.hpp) of every block with precondition_min_k
+  // QR preconditioning (precond.hpp), one pass: a second one over the columns
+  // at the Gram matrix's resolution empties a null space sooner (38 against 45 ms
+  // at 2000 multiplets) but leaves its values ten times below those of other
+  // sectors, and a run that keeps more multiplets than its state has fills up
+  // with directions of the wrong sectors (first 16x8 sweeps up to 12 % above
+  // the usual energy).
+  // Every block with precondition_min_k
   // <= K <= kPrecondMaxK: columns sorted, then W <- W P Q2 and V <- P Q2.  A block's
   // own size decides, so its bits do not depend on the rest of the batch (a
   // block left out is sorted here instead of at the first sweep: the same
@@ -1350,7 +1349,7 @@ static int jacobi_svd_large(Context& c, const std::vector<JacobiBlock*>& blocks,
     if (!pre.empty()) {
       sort_permute(nullptr);
       for (int b : pre)
-        pb.push_back(PrecondBlock{Wc[b], Vc[b], Wo[b], Vo[b], L[b], K[b], K[b], desc[b].normF, 0.0});
+        pb.push_back(PrecondBlock{Wc[b], Vc[b], Wo[b], Vo[b], L[b], K[b], desc[b].normF});
       precondition_jacobi(c, pb, plain);
       for (int b : pre) {
         std::swap(Wc[b], Wo[b]);
@@ -1358,38 +1357,6 @@ static int jacobi_svd_large(Context& c, const std::vector<JacobiBlock*>& blocks,
       }
       upload();
       norms();
-      // The Gram matrix resolves directions down to 3e-8 of the block; the
-      // columns below that are still a mixture of everything under it.
-      // They are preconditioned among themselves, with their own Gram matrix
-      // (which resolves 3e-8 of theirs), so that the null space drops to the
-      // rounding level at once and leaves the sweeps.
-      if (!plain) sort_permute(nullptr);
-      std::vector<PrecondBlock> tail;
-      std::vector<VecMove> back;
-      for (const int b : plain ? std::vector<int>() : pre) {
-        const double thr = kTailRel * desc[b].normF * (kTailRel * desc[b].normF);
-        int r = 0;
-        while (r < K[b] && hn[noff[b] + r] > thr) ++r;
-        const int n = K[b] - r;
-        if (n < kTailMin) continue;
-        double top = 0.0, sum = 0.0;
-        for (int q = r; q < K[b]; ++q) {
-          const double w = hn[noff[b] + q];
-          top = std::max(top, w);
-          sum += w;
-        }
-        if (!(std::sqrt(top) > kNoiseRel * desc[b].normF)) continue;
-        const long long wo = (long long)r * L[b], vo = (long long)r * K[b];
-        tail.push_back(PrecondBlock{Wc[b] + wo, Vc[b] + vo, Wo[b] + wo, Vo[b] + vo, L[b], n, K[b],
-                                    std::sqrt(sum), kTailNoise * desc[b].normF});
-        back.push_back(VecMove{Wo[b] + wo, Wc[b] + wo, (long long)n * L[b], kMoveF64, 0});
-        back.push_back(VecMove{Vo[b] + vo, Vc[b] + vo, (long long)n * K[b], kMoveF64, 0});
-      }
-      if (!tail.empty()) {
-        precondition_jacobi(c, tail, false);
-        dev_moves(c, back);
-      }
-      if (!tail.empty()) norms();
     }
   }
   // Deflation: the columns of a block above the rounding level, kept[b] of

@@ -605,7 +605,7 @@ void precondition_jacobi(Context& c, std::vector<PrecondBlock>& blocks, bool pla
     off += 2 * kk + np * PB * PB;
     d.K = b.K;
     d.rk = b.K;
-    d.tiny = std::max(1e-15 * b.normF * b.normF, b.noise * b.noise);
+    d.tiny = 1e-15 * b.normF * b.normF;
   }
   DevBuf ddesc(c, (long long)((sizeof(PDesc) * nb + 7) / 8));
   SU2_HIP(hipMemcpyAsync(ddesc.p, hd.data(), sizeof(PDesc) * nb, hipMemcpyHostToDevice, st));
@@ -666,7 +666,7 @@ void precondition_jacobi(Context& c, std::vector<PrecondBlock>& blocks, bool pla
     for (int i = 0; i < nb; ++i) {
       const PrecondBlock& b = blocks[i];
       g.add(b.Wout, b.L, b.L, b.K, b.W, b.L, 0, hd[i].Q, b.K, 0, b.K);
-      g.add(b.Vout, b.VR, b.VR, b.K, b.V, b.VR, 0, hd[i].Q, b.K, 0, b.K);
+      g.add(b.Vout, b.K, b.K, b.K, b.V, b.K, 0, hd[i].Q, b.K, 0, b.K);
     }
     g.run(c);
   }

@@ -28,12 +28,12 @@ class Context;
 
 struct PrecondBlock {
   const double* W;  // L x K, ld L
-  const double* V;  // VR x K, ld VR
+  const double* V;  // K x K
   double* Wout;     // L x K, ld L: receives W Q2
-  double* Vout;     // VR x K, ld VR: receives V Q2
-  int L, K, VR;
+  double* Vout;     // K x K: receives V Q2
+  int L, K;
   double normF;     // Frobenius norm of W; a Cholesky pivot at or below 1e-15 normF^2
-  double noise;     // or noise^2 (rounding errors of W's columns) gives a zero row
+                    // gives a zero row
 };
 
 // Largest K the panel kernels take (two rows per thread of 1024, held in

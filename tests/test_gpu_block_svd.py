@@ -3,8 +3,7 @@
 Such calls take the preconditioned block Jacobi (an uncut call keeps the plain iteration, which
 test_gpu_dmrg covers): pairs of 32-column blocks rotated against each other, whole blocks in their
 first visit of a sweep, only the pairs that still need it.  Sizes just past the LDS limit, a last
-column block of one column, a block far taller than wide, and rank-deficient ones whose null space
-a second preconditioning pass removes; both column block widths and up to three inner sweeps.
+column block of one column, a block far taller than wide, and rank-deficient ones; both column block widths and up to three inner sweeps.
 """
 import sys
 
