@@ -345,8 +345,9 @@ int su2_dmrg_set_matvec_precision(su2_ctx* ctx, su2_dmrg* d, int bits, double mi
  * For measurements on the real state (energy, variance, hermiticity) and
  * timing the matvec on the run's own sector dimensions. */
 int su2_dmrg_centre(su2_ctx* ctx, su2_dmrg* d, su2_heff** plan, su2_tensor** psi);
-/* H_eff launches of each solve replayed from a HIP graph (on = 1, default)
- * or launched directly (0); the results are the same. */
+/* H_eff launches of each solve replayed from a HIP graph where several solves
+ * share them (on = 1, default) or always launched directly (0); the results
+ * are the same. */
 int su2_dmrg_set_graph(su2_ctx* ctx, su2_dmrg* d, int on);
 
 /* Several DMRG runs of one context advanced in lockstep (no counterpart in

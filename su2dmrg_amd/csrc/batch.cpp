@@ -88,6 +88,7 @@ HeffBatch::Pattern& HeffBatch::pattern(const std::vector<Req>& reqs) {
       P->run2.push_back(&P->s2[pi]);
     }
   }
+  P->lone = reqs.size() == 1;
   Pattern& ref = *P;
   cache_[key] = std::move(P);
   return ref;
@@ -129,7 +130,10 @@ void HeffBatch::apply(const std::vector<Req>& reqs) {
     outs.push_back(out);
   }
   dev_moves(c_, ins);
-  if (!use_graph_) {
+  // A replay costs the host 15 to 25 us and its recording 50 us a list of
+  // requests (one per solve for a lone run), a launch 3 us: a 6x4 run up to
+  // d = 924 took 241 ms with every round replayed and takes 236.
+  if (!use_graph_ || P.lone) {
     launch_body(P);
   } else {
     if (!P.exec) {

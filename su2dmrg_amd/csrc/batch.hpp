@@ -52,11 +52,12 @@ class HeffBatch {
   // y_i = H_i x_i for every request (plans must stay alive while this
   // object caches launches for them; call clear() before destroying plans).
   // The first apply for a given list of (plan, precision) builds its grouped
-  // launches and captures them in a HIP graph; later applies for the same
-  // list replay that graph with new x and y.  Does not wait.
+  // launches and, for several requests, captures them in a HIP graph; later
+  // applies for the same list replay it with new x and y.  A lone request's
+  // two to five launches go out directly.  Does not wait.
   void apply(const std::vector<Req>& reqs);
   void clear();
-  // Use the graph (default) or launch the same kernels directly.
+  // Use graphs (default) or launch the same kernels directly.
   void set_use_graph(bool on) { use_graph_ = on; }
   int graphs_built() const { return graphs_built_; }
   long long replays() const { return replays_; }
@@ -67,6 +68,7 @@ class HeffBatch {
     // what a launch runs: the above, or a single request's own plans
     std::vector<const GroupedGemm*> run1, run2;
     std::vector<VecMove> fill;  // zero blocks of the outputs (fixed)
+    bool lone = false;          // one request
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     Pattern() : s1{GroupedGemm(Prec::F64), GroupedGemm(Prec::F32)},
