@@ -331,10 +331,12 @@ __global__ __launch_bounds__(kThreads, 1) void small_svd_kernel(const SmallArgs 
     double best = max16(fmax(tagged(n0, lane), tagged(n1, 64 + lane)));
     best = fmax(fmax(lane_value(best, 0), lane_value(best, 16)),
                 fmax(lane_value(best, 32), lane_value(best, 48)));
-    // the remaining columns are at the rounding level of the block: nothing to order
-    if (!(best > 1e-4 * noise2)) break;
+    // the remaining columns are at the rounding level of the block: nothing to order.  The exact
+    // norm decides where that level underflows: the row in the low bits of `best` makes a norm of
+    // zero positive, and the reciprocals below take normal numbers only.
     const int piv = tag_of(best);
     const double nn = lane_value(piv >= 64 ? n1 : n0, piv % 64);
+    if (!(best > 1e-4 * noise2) || !(nn >= 0x1p-1022)) break;
     const double alpha = X[i * ld + piv];
     const double beta = -copysign(nn * rsqrt_of(nn), alpha);
     const double tau = (beta - alpha) * recip_signed(beta), scale = recip_signed(alpha - beta);
