@@ -41,6 +41,8 @@ constexpr int kMaxL = 128;
 constexpr int kColChunk = 8;      // columns a wave loads at once for a reflector
 // 160 KB of LDS per CU, less the small arrays
 constexpr int kLdsDoubles = 20480 - 2 * kThreads - 3 * kMaxK;
+// elements of the block per thread (W is half of the LDS array at most)
+constexpr int kElems = (kLdsDoubles / 2 + kThreads - 1) / kThreads;
 
 typedef double f64x2 __attribute__((ext_vector_type(2)));
 
@@ -281,17 +283,58 @@ __global__ __launch_bounds__(kThreads, 1) void small_svd_kernel(const SmallArgs 
   const int G = pair_lanes(k), NW = row_pairs(L, k), Lp = 2 * G * NW, rows = 2 * Lp;
   const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
 
-  // W (the block, transposed when it is wider than tall), V = 1, zeros in the padding
+  // W (the block, transposed when it is wider than tall), V = 1, their columns in one order, zeros
+  // in the padding
   for (int e = t; e < ld * k; e += kThreads) X[e] = 0.0;
   if (t < 2) s_worst[t] = 0ull;
   __syncthreads();
-  for (int e = t; e < D.m * D.n; e += kThreads) {
-    const int r = e % D.m, c = e / D.m;
-    const double v = D.A[e];
-    if (D.m >= D.n) X[c * ld + r] = v;
-    else X[r * ld + c] = v;
+  // the block's elements, by way of registers (their order in LDS is not known yet)
+  const int total = D.m * D.n;
+  double a[kElems];
+#pragma unroll
+  for (int i = 0; i < kElems; ++i) {
+    if (kThreads * i >= total) break;
+    const int e = t + kThreads * i;
+    a[i] = e < total ? D.A[e] : 0.0;
   }
-  for (int c = t; c < k; c += kThreads) X[c * ld + Lp + c] = 1.0;
+  auto place = [&](auto column) {
+    int r = t % D.m, c = t / D.m;
+    const int dr = kThreads % D.m, dc = kThreads / D.m;
+#pragma unroll
+    for (int i = 0; i < kElems; ++i) {
+      if (kThreads * i >= total) break;
+      if (t + kThreads * i < total) {
+        if (D.m >= D.n) X[column(c) * ld + r] = a[i];
+        else X[column(r) * ld + c] = a[i];
+      }
+      r += dr;
+      c += dc;
+      if (r >= D.m) {
+        r -= D.m;
+        ++c;
+      }
+    }
+  };
+  // Columns by descending norm.  A Householder QR of W^T with pivoting (the reflectors below) is
+  // then backward stable column by column of W as well, after Cox and Higham, and values far below
+  // the largest keep their relative accuracy where W's columns span many decades: 48 shuffled
+  // columns over six decades lost 2e-11 of the smallest values unsorted and lose 2e-15.
+  place([](int c) { return c; });
+  __syncthreads();
+  column_norms<4>(X, k, ld, 0, Lp / 8, t, s_norm);
+  __syncthreads();
+  for (int c = t; c < k; c += kThreads) {
+    const double v = s_norm[c];
+    int pos = 0;   // ties by column, NaN first
+    for (int d = 0; d < k; ++d) {
+      const double u = s_norm[d];
+      pos += u != u ? v == v || d < c : u > v || (u == v && d < c);
+    }
+    s_pos[c] = pos;
+    X[pos * ld + Lp + c] = 1.0;
+  }
+  __syncthreads();
+  place([&](int c) { return s_pos[c]; });
   __syncthreads();
 
   // ---- Householder reflectors from the right ----
