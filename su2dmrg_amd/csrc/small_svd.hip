@@ -544,8 +544,11 @@ int small_svd_batched(Context& c, const std::vector<JacobiBlock*>& blocks, doubl
     lds = std::max(lds, sizeof(double) * (size_t)desc[i].ld * k);
   }
   double* host = c.host_scratch(tot);
+  // the most any launch takes, and not this one's need: the attribute is the
+  // kernel's, and another context's thread may set it before this launch
   SU2_HIP(hipFuncSetAttribute((const void*)small_svd_kernel,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+                              hipFuncAttributeMaxDynamicSharedMemorySize,
+                              (int)(sizeof(double) * kLdsDoubles)));
   for (int i0 = 0; i0 < nb; i0 += kBlocksPerLaunch) {
     SmallArgs args;
     const int n = std::min(kBlocksPerLaunch, nb - i0);
