@@ -782,7 +782,7 @@ __device__ __forceinline__ void pair_sweeps(const PairLds& S, int n, double fl,
 // Diagonalises one pair's Gram matrix: the slices' partial sums in slice
 // order, the convergence test, then inner_sweeps sweeps of parallel cyclic
 // Jacobi in LDS, and the accumulated rotation to rot (column-major, NP rows).
-// *active says whether the pair rotated at all.
+// *active says whether the pair rotated at all; *moved is set if it did.
 //
 // A pair rotates its p columns against its q columns only (CB rounds of CB
 // disjoint rotations): the pairs inside a block are rotated in the block's
@@ -808,7 +808,8 @@ template <int CB>
 __device__ __forceinline__ void solve_pair(const BlockDesc& B, const PairJob& J,
                                            const double* __restrict__ gp, double tol_rel,
                                            double tol_abs, int inner_sweeps, double* lds,
-                                           double* __restrict__ rot, int* __restrict__ active) {
+                                           double* __restrict__ rot, int* __restrict__ active,
+                                           int* __restrict__ moved) {
   constexpr int NP = 2 * CB, TT = NP / 16, NU = TT * (TT + 1) / 2, NT = SolveThreads<CB>::value;
   double* G = lds;                       // NP x NP, upper triangle
   double* R = G + NP * NP;               // R[column][row]
@@ -860,7 +861,10 @@ __device__ __forceinline__ void solve_pair(const BlockDesc& B, const PairJob& J,
     }
   }
   const bool any = __syncthreads_or(need);
-  if (t == 0) *active = any;
+  if (t == 0) {
+    *active = any;
+    if (any) *moved = 1;
+  }
   if (!any) return;
 
   PairLds L{G, R, cs, tn, rotated};
@@ -915,19 +919,21 @@ __device__ __forceinline__ void apply_rows(double* __restrict__ M, int rows, con
 
 // The first nj workgroups diagonalise this round's pairs, the others apply
 // the previous round's rotations to V's row tiles (nv of them per pair).
+// moved: one flag per block of the batch (pinned), set where a pair rotated.
 template <int CB>
 __global__ __launch_bounds__(SolveThreads<CB>::value) void solve_kernel(
     const BlockDesc* __restrict__ blocks, const PairJob* __restrict__ jobs, int nj, int pmax,
     const double* __restrict__ gpart, double tol_rel, double tol_abs, int inner_sweeps,
-    double* __restrict__ rot, int* __restrict__ active, const PairJob* __restrict__ vjobs, int nv,
-    const double* __restrict__ vrot, const int* __restrict__ vactive) {
+    double* __restrict__ rot, int* __restrict__ active, int* __restrict__ moved,
+    const PairJob* __restrict__ vjobs, int nv, const double* __restrict__ vrot,
+    const int* __restrict__ vactive) {
   constexpr int NP = 2 * CB, NU = (NP / 16) * (NP / 16 + 1) / 2;
   __shared__ __align__(16) double lds[2 * NP * NP + 6 * CB + 2];
   const int i = blockIdx.x;
   if (i < nj) {
     const PairJob J = jobs[i];
     solve_pair<CB>(blocks[J.blk], J, gpart + (size_t)i * pmax * NU * 256, tol_rel, tol_abs,
-                   inner_sweeps, lds, rot + (size_t)i * NP * NP, active + i);
+                   inner_sweeps, lds, rot + (size_t)i * NP * NP, active + i, moved + J.blk);
     return;
   }
   const int job = (i - nj) / nv, tile = (i - nj) - job * nv;
@@ -1654,8 +1660,8 @@ static int jacobi_svd_large(Context& c, const std::vector<JacobiBlock*>& blocks,
     const int rows_per_tile = (CB == 32 ? SolveThreads<32>::value : SolveThreads<16>::value) / 4;
     const int wt = (lmax + rows_per_tile - 1) / rows_per_tile;
     const int vt = (kmax + rows_per_tile - 1) / rows_per_tile;
-    // one round's three launches; round -1 of the next call: only V's rotations
-    auto run_rounds = [&](auto cb) {
+    // each round's three launches, and a last one for V's rotations of the last round
+    auto run_rounds = [&](auto cb, int* moved) {
       constexpr int B = decltype(cb)::value;
       constexpr int NT = SolveThreads<B>::value;
       const BlockDesc* dd = ddesc;
@@ -1680,7 +1686,7 @@ static int jacobi_svd_large(Context& c, const std::vector<JacobiBlock*>& blocks,
         if (nj + nprev > 0)
           hipLaunchKernelGGL(solve_kernel<B>, dim3(nj + nprev * vt), dim3(NT), 0, st, dd, jr, nj,
                              pm, (const double*)dgpart.p, tol, kTolAbs, inner_sweeps, rot, act,
-                             prev, vt, prot, pact);
+                             moved, prev, vt, prot, pact);
         if (nj > 0)
           hipLaunchKernelGGL(apply_kernel<B>, dim3(nj * wt), dim3(NT), 0, st, dd, jr, wt,
                              (const double*)rot, (const int*)act);
@@ -1698,9 +1704,17 @@ static int jacobi_svd_large(Context& c, const std::vector<JacobiBlock*>& blocks,
       converged = all.empty();
       if (converged || sweep == max_sweeps) break;
       ++sweeps_done;
-      if (CB == 16) run_rounds(std::integral_constant<int, 16>{});
-      else run_rounds(std::integral_constant<int, 32>{});
+      // The solve launches test every scheduled pair again, on Gram matrices
+      // summed in another order.  A pair at the threshold can pass there, so a
+      // block whose pairs all passed is done: nothing would change in the next
+      // sweep, nor its flags.
+      int* moved = (int*)(c.host_scratch(2 * ncol + nb) + 2 * ncol);
+      std::fill(moved, moved + nb, 0);
+      if (CB == 16) run_rounds(std::integral_constant<int, 16>{}, moved);
+      else run_rounds(std::integral_constant<int, 32>{}, moved);
       norms();
+      for (int b = 0; b < nb; ++b)
+        if (!moved[b]) active[b] = 0;
     }
   }
   // Out of sweeps: the columns are accepted when orthogonal to 1e-6 of their
