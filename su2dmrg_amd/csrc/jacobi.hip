@@ -24,10 +24,6 @@ namespace {
 constexpr int INNER_SWEEPS = 3; // most inner Jacobi sweeps per visit of a pair
 constexpr int MAX_SLICES = 8;   // row slices per pair
 constexpr int MIN_SLICE_ROWS = 64;
-// Columns with norm at or below kNoiseRel ||A||_F are at the rounding level
-// of the block: they carry no direction, no pair with one of them holds the
-// iteration open, and the sweeps leave them out of the schedule.
-constexpr double kNoiseRel = 1e-13;
 // Blocks under this many columns are preconditioned whatever the setting says:
 // a 192 x 192 block takes 5.5 ms that way and 14.4 ms without.
 constexpr int kPrecondAlways = 256;

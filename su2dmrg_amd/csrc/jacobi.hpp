@@ -37,7 +37,7 @@
 // Sweeps stop when every pair is orthogonal to
 // |g_ij| <= max(tol * sqrt(g_ii g_jj), 1e-14 ||A||_F (sqrt g_ii + sqrt g_jj))
 // (the absolute floor ends the iteration on columns that carry rounding
-// errors of order eps ||A||); columns with norm <= 1e-13 ||A||_F are left
+// errors of order eps ||A||); columns with norm <= kNoiseRel ||A||_F are left
 // out of the test.
 #pragma once
 
@@ -46,6 +46,11 @@
 namespace su2 {
 
 class Context;
+
+// Columns with norm at or below kNoiseRel ||A||_F are at the rounding level of
+// the block: they carry no direction, no pair with one of them holds the
+// iteration open, and the sweeps leave them as they are.
+constexpr double kNoiseRel = 1e-13;
 
 struct JacobiBlock {
   const double* A;   // m x n, column-major, leading dimension m (device)

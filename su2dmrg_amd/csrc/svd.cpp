@@ -67,18 +67,46 @@ void svd_values(std::vector<Sec>& secs, std::vector<std::vector<double>>& wv, do
   }
 }
 
+// Order of a sector's values in the global cut: the values themselves, except
+// those at the rounding level of the sector.  A null direction's value is
+// whatever its kernel left (1e-14 to 6e-14 of the sector's norm in blocks past
+// one compute unit's LDS, 1e-16 in smaller ones), and by that the cut would
+// take all null directions of some sectors before any of others.  A run that
+// keeps more multiplets than its state has grows into the null directions it
+// kept: over 51 runs of 16x8 and 12x6 cylinders at D = 220 to 650, the second
+// sweep ended above that of one kernel for every size in 37, with the levels
+// here in 25.  The null values of a sector are therefore spread evenly up to
+// kNullLevel of its norm, which gives sectors of equal norm the same fraction.
+constexpr double kNullLevel = 4e-14;
+
+std::vector<double> cut_keys(const std::vector<double>& s) {
+  double norm = 0;
+  for (double x : s) norm += x * x;
+  norm = std::sqrt(norm);
+  std::vector<double> key = s;
+  std::vector<size_t> null;
+  for (size_t t = 0; t < s.size(); ++t)
+    if (s[t] > 0 && s[t] <= kNoiseRel * norm) null.push_back(t);
+  for (size_t i = 0; i < null.size(); ++i)
+    key[null[i]] = kNullLevel * norm * ((double)i + 0.5) / (double)null.size();
+  return key;
+}
+
 // Global cut and output tensors of one wavefunction; the kept columns times
 // their factors go to `outs`, which fill every element of both tensors.
 SvdResult svd_cut(Context& c, const Tensor& psi, std::vector<Sec>& secs, int max_dcut,
                   const double* dfac, const std::vector<long long>& foff,
                   std::vector<ScaledColumns>& outs) {
-  std::vector<double> wsort;
-  std::vector<int> isort;
+  std::vector<double> wsort, val;   // sort keys; the values they stand for
+  std::vector<int> isort, sec;
   for (size_t i = 0; i < secs.size(); ++i) {
     const Sec& s = secs[i];
-    for (int t = 0; t < s.dc; ++t) {
-      wsort.push_back(s.s[s.k - s.dc + t]);
-      isort.push_back((int)i);
+    const std::vector<double> key = cut_keys(s.s);
+    for (int t = s.k - s.dc; t < s.k; ++t) {
+      wsort.push_back(key[t]);
+      isort.push_back((int)val.size());
+      val.push_back(s.s[t]);
+      sec.push_back((int)i);
     }
   }
   // global cut: shell sort ascending, keep the top max_dcut
@@ -86,9 +114,9 @@ SvdResult svd_cut(Context& c, const Tensor& psi, std::vector<Sec>& secs, int max
   const int ntot = (int)wsort.size();
   const int k0 = max_dcut > ntot ? 0 : ntot - max_dcut;
   std::vector<int> keep(secs.size(), 0);
-  for (int t = ntot - 1; t >= k0; --t) keep[isort[t]]++;
+  for (int t = ntot - 1; t >= k0; --t) keep[sec[isort[t]]]++;
   double disc = 0;
-  for (int t = 0; t < k0; ++t) disc += wsort[t] * wsort[t];
+  for (int t = 0; t < k0; ++t) disc += val[isort[t]] * val[isort[t]];
 
   SvdResult res;
   std::vector<int> bt, bd;
