@@ -87,8 +87,9 @@ int su2_ctx_set_svd_tuning(su2_ctx* ctx, int block_cols, int inner_sweeps);
  * and a rank-deficient one (two-site wavefunction sectors typically are)
  * has its null directions in columns at the rounding level from the start,
  * which the sweeps leave out: a 16x8 D=2000 sweep takes about 26 s instead
- * of 37 s.  Blocks of fewer than 256 columns are always preconditioned, again
- * unless nothing can be cut.
+ * of 37 s.  A limit of up to 256, the default among them, also preconditions
+ * the smaller blocks past one compute unit's LDS, unless nothing can be cut
+ * (su2_svd_truncate); 0 and limits above 256 hold as given.
  * The reference computes its sector SVDs through the Gram matrix and dsyev
  * (tensor.cpp:1472-1529); this setting changes results by rounding only. */
 int su2_ctx_set_svd_precondition(su2_ctx* ctx, int min_k);

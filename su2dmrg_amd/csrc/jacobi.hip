@@ -24,9 +24,10 @@ namespace {
 constexpr int INNER_SWEEPS = 3; // most inner Jacobi sweeps per visit of a pair
 constexpr int MAX_SLICES = 8;   // row slices per pair
 constexpr int MIN_SLICE_ROWS = 64;
-// Blocks under this many columns are preconditioned whatever the setting says:
-// a 192 x 192 block takes 5.5 ms that way and 14.4 ms without.
-constexpr int kPrecondAlways = 256;
+// A limit up to this many columns, the default among them, preconditions the
+// smaller blocks as well: a 192 x 192 block takes 5.5 ms that way and 14.4 ms
+// without.
+constexpr int kPrecondDefault = 256;
 constexpr double kTolAbs = 1e-14;   // rounding floor of a pair, relative to ||A||_F
 
 typedef double f64x4 __attribute__((ext_vector_type(4)));
@@ -1335,19 +1336,17 @@ static int jacobi_svd_large(Context& c, const std::vector<JacobiBlock*>& blocks,
   // sectors, and a run that keeps more multiplets than its state has fills up
   // with directions of the wrong sectors (first 16x8 sweeps up to 12 % above
   // the usual energy).
-  // Every block with precondition_min_k
-  // <= K <= kPrecondMaxK: columns sorted, then W <- W P Q2 and V <- P Q2.  A block's
-  // own size decides, so its bits do not depend on the rest of the batch (a
-  // block left out is sorted here instead of at the first sweep: the same
+  // Columns sorted, then W <- W P Q2 and V <- P Q2.  A block's own size and the
+  // setting decide, so its bits do not depend on the rest of the batch (a block
+  // left out is sorted here instead of at the first sweep: the same
   // permutation, and the first sweep's sort is then the identity).
   {
     std::vector<PrecondBlock> pb;
     std::vector<int> pre;
     for (int b = 0; b < nb; ++b)
-      if ((!plain && K[b] < kPrecondAlways) ||
-          (precondition_min_k > 0 && K[b] >= precondition_min_k && K[b] <= kPrecondMaxK)) {
+      if (precondition_min_k > 0 && K[b] <= kPrecondMaxK &&
+          (K[b] >= precondition_min_k || (!plain && precondition_min_k <= kPrecondDefault)))
         pre.push_back(b);
-      }
     if (!pre.empty()) {
       sort_permute(nullptr);
       for (int b : pre)

@@ -172,7 +172,8 @@ class Context:
 
     def set_svd_precondition(self, min_k=256):
         """QR preconditioning of the Jacobi SVD for sector blocks with
-        min(m, n) >= min_k (the context's default is 256; 0 or False: off;
+        min(m, n) >= min_k (the context's default is 256, which takes the
+        smaller blocks along where a cut is possible; 0 or False: off;
         True: 256)."""
         if min_k is True:
             min_k = 256
