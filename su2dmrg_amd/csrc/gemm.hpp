@@ -95,11 +95,13 @@ class GroupedGemm {
   // Re-tiles for another variant (device tables rebuilt) and keeps it.
   void set_variant(int v);
   int variant() const { return variant_; }
+  // The tables anew for the same variant, pinned or not (after allow_uniform).
+  void rebuild() { build(variant_); }
   // the variant that set_variant (or autotune) asked for, -1 if none did
   int pinned_variant() const { return pinned_ ? variant_ : -1; }
   // Launches whose slices share one layout (op(B) = B, op(A) fixed) run the
   // straight-line uniform kernel unless this is switched off (before
-  // finalize or set_variant); layout() is 0 (NN), 1 (TN) or -1 (mixed).
+  // finalize, set_variant or rebuild); layout() is 0 (NN), 1 (TN) or -1 (mixed).
   void allow_uniform(bool on) { uniform_ = on; }
   int layout() const { return layout_; }
   // Times every variant (HIP events, `reps` launches each) and keeps the

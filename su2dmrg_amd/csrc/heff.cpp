@@ -341,7 +341,7 @@ void HeffPlan::set_uniform(bool on) {
   ctx_.make_current();
   for (int i = 0; i < 2; ++i) {
     stage(i).allow_uniform(on);
-    stage(i).set_variant(stage(i).variant());
+    stage(i).rebuild();
   }
 }
 
