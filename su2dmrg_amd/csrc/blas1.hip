@@ -2,6 +2,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <memory>
 #include <mutex>
 
 #include "common.hpp"
@@ -141,7 +142,13 @@ __global__ void axpy_dev_kernel(double* __restrict__ y, const double* __restrict
   for (; i < n; i += stride) y[i] += av * x[i];
 }
 
-constexpr int kAxpyChunk = 1024;   // elements of one group per workgroup
+// Elements of one group per workgroup.  Small groups are bound by latency and
+// take short chunks; a group that fills the chip either way takes long ones,
+// since the host writes and uploads 16 bytes for each: the scatters of two
+// 16x8 D = 2000 sweeps took it 280 ms with 1024 throughout, 70 ms now (with
+// tables written once; 130 ms without that).
+constexpr int kAxpyChunk = 1024, kAxpyChunkLong = 4096;
+constexpr long long kAxpyLong = 1 << 16;
 
 // nsum consecutive descriptors from desc on (the bundle kernel's chunks name
 // one descriptor, and how it is walked in nsum)
@@ -460,47 +467,53 @@ void dev_axpy_dev(Context& c, double* y, const double* x, long long n, const dou
   SU2_HIP(hipGetLastError());
 }
 
-void dev_strided_axpy_launches(Context& c,
-                               const std::vector<std::vector<StridedSum>>& launches) {
-  std::vector<StridedAxpy> flat;
-  std::vector<AxpyChunk> chunks;
-  std::vector<TileRef> tiles;
-  // chunk and tile ranges of each launch
+void dev_strided_sums(Context& c, const std::vector<StridedAxpy>& desc,
+                      const std::vector<StridedSum>& groups, const std::vector<int>& ends) {
+  auto tiled = [](const StridedAxpy& d) {
+    return d.src && d.cs == 1 && d.rs > 1 && d.rows > 1 && d.cols > 1;
+  };
+  auto per_chunk = [](long long n) { return n < kAxpyLong ? kAxpyChunk : kAxpyChunkLong; };
+  // chunk and tile ranges of each launch; the tables are then written where
+  // they are uploaded from
   std::vector<std::pair<size_t, size_t>> span, tspan;
-  for (auto& l : launches) {
-    const size_t c0 = chunks.size(), t0 = tiles.size();
-    for (const StridedSum& g : l) {
-      if (g.empty()) continue;
-      const StridedAxpy& d = g[0];
+  size_t nc = 0, nt = 0;
+  int g = 0;
+  for (int end : ends) {
+    const size_t c0 = nc, t0 = nt;
+    for (; g < end; ++g) {
+      const StridedAxpy& d = desc[groups[g].first];
       const long long n = (long long)d.rows * d.cols;
-      if (n <= 0) continue;
       SU2_CHECK(n < (1LL << 31), kErrCapacity, "strided axpy: block of %lld elements", n);
-      const int di = (int)flat.size(), ns = (int)g.size();
-      flat.insert(flat.end(), g.begin(), g.end());
-      if (d.src && d.cs == 1 && d.rs > 1 && d.rows > 1 && d.cols > 1) {
-        for (int cc = 0; cc < d.cols; cc += kTile)
-          for (int r0 = 0; r0 < d.rows; r0 += kTile) tiles.push_back(TileRef{di, r0, cc, ns});
-      } else {
-        for (long long f = 0; f < n; f += kAxpyChunk)
-          chunks.push_back(AxpyChunk{di, (int)f, (int)std::min<long long>(kAxpyChunk, n - f), ns});
-      }
+      if (tiled(d)) nt += (size_t)((d.cols + kTile - 1) / kTile) * ((d.rows + kTile - 1) / kTile);
+      else nc += (n + per_chunk(n) - 1) / per_chunk(n);
     }
-    span.push_back({c0, chunks.size()});
-    tspan.push_back({t0, tiles.size()});
+    span.push_back({c0, nc});
+    tspan.push_back({t0, nt});
   }
-  if (chunks.empty() && tiles.empty()) return;
-  SU2_CHECK(tiles.size() < (1u << 31), kErrCapacity, "strided axpy: %zu tiles", tiles.size());
-  const size_t dbytes = (flat.size() * sizeof(StridedAxpy) + 15) / 16 * 16;
-  const size_t cbytes = (chunks.size() * sizeof(AxpyChunk) + 15) / 16 * 16;
-  const size_t bytes = dbytes + cbytes + tiles.size() * sizeof(TileRef);
-  std::vector<char> host(bytes, 0);
-  std::memcpy(host.data(), flat.data(), flat.size() * sizeof(StridedAxpy));
-  if (!chunks.empty())
-    std::memcpy(host.data() + dbytes, chunks.data(), chunks.size() * sizeof(AxpyChunk));
-  if (!tiles.empty())
-    std::memcpy(host.data() + dbytes + cbytes, tiles.data(), tiles.size() * sizeof(TileRef));
+  if (nc + nt == 0) return;
+  SU2_CHECK(nt < (1u << 31) && nc < (1u << 31), kErrCapacity,
+            "strided axpy: %zu tiles, %zu chunks", nt, nc);
+  const size_t dbytes = (desc.size() * sizeof(StridedAxpy) + 15) / 16 * 16;
+  const size_t cbytes = (nc * sizeof(AxpyChunk) + 15) / 16 * 16;
+  const size_t bytes = dbytes + cbytes + nt * sizeof(TileRef);
+  const std::unique_ptr<char[]> host(new char[bytes]);
+  std::memcpy(host.get(), desc.data(), desc.size() * sizeof(StridedAxpy));
+  AxpyChunk* chunk = (AxpyChunk*)(host.get() + dbytes);
+  TileRef* tile = (TileRef*)(host.get() + dbytes + cbytes);
+  for (const StridedSum& s : groups) {
+    const StridedAxpy& d = desc[s.first];
+    if (tiled(d)) {
+      for (int cc = 0; cc < d.cols; cc += kTile)
+        for (int r0 = 0; r0 < d.rows; r0 += kTile) *tile++ = TileRef{s.first, r0, cc, s.count};
+    } else {
+      const long long n = (long long)d.rows * d.cols;
+      const int per = per_chunk(n);
+      for (long long f = 0; f < n; f += per)
+        *chunk++ = AxpyChunk{s.first, (int)f, (int)std::min<long long>(per, n - f), s.count};
+    }
+  }
   char* dev = (char*)c.dev_alloc(bytes);
-  SU2_HIP(hipMemcpyAsync(dev, host.data(), bytes, hipMemcpyHostToDevice, c.stream()));
+  SU2_HIP(hipMemcpyAsync(dev, host.get(), bytes, hipMemcpyHostToDevice, c.stream()));
   const StridedAxpy* d_desc = (const StridedAxpy*)dev;
   const AxpyChunk* d_chunks = (const AxpyChunk*)(dev + dbytes);
   const TileRef* d_tiles = (const TileRef*)(dev + dbytes + cbytes);

@@ -63,16 +63,20 @@ struct StridedAxpy {
   int rows, cols;   // rows * cols < 2^31
   double alpha;
 };
-// Descriptors of one group share destination, strides and shape (and whether
-// they have a source); their terms are added one after the other, in order.
-typedef std::vector<StridedAxpy> StridedSum;
-// One launch per inner vector of groups, in order on the context stream (a
-// later launch may add into what an earlier one wrote); the descriptors of
-// all launches are uploaded together and the call does not wait.  Every group
-// is cut into chunks of up to kAxpyChunk elements, one workgroup each, so a
+// Descriptors first .. first + count - 1 of one group share destination,
+// strides and shape (and whether they have a source); their terms are added
+// one after the other, in order.
+struct StridedSum {
+  int first, count;
+};
+// groups[ends[i - 1]] .. groups[ends[i] - 1] go to launch i, the launches in
+// order on the context stream (a later launch may add into what an earlier one
+// wrote); the descriptors of all launches are uploaded together and the call
+// does not wait.  Every group is cut into chunks, one workgroup each, so a
 // workgroup reads its descriptors once and indexes with 32-bit arithmetic,
 // and an element is read and written once however many terms it has.
-void dev_strided_axpy_launches(Context& c, const std::vector<std::vector<StridedSum>>& launches);
+void dev_strided_sums(Context& c, const std::vector<StridedAxpy>& desc,
+                      const std::vector<StridedSum>& groups, const std::vector<int>& ends);
 
 // Operator bundles: each descriptor holds nt summands of rows x cols
 // column-major blocks, element q = r + rows*c of summand t written once as

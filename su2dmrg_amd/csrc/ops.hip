@@ -53,24 +53,47 @@ void GemmBatch::run(Context& c, int variant) {
 
 void ScatterBatch::add(const void* key, const StridedAxpy& d) {
   if (d.rows <= 0 || d.cols <= 0) return;
-  auto it = last_.find(key);
+  const int id = (int)entries_.size();
+  entries_.push_back(Entry{d, -1});
+  const auto it = last_.emplace(key, (int)groups_.size());
   int launch = 0;
-  if (it != last_.end()) {
-    StridedSum& g = launches_[it->second.first][it->second.second];
-    const StridedAxpy& h = g[0];
+  if (!it.second) {
+    Group& g = groups_[it.first->second];
+    const StridedAxpy& h = entries_[g.first].d;
     if (h.dst == d.dst && h.rs == d.rs && h.cs == d.cs && h.rows == d.rows && h.cols == d.cols &&
         (h.src != nullptr) == (d.src != nullptr)) {
-      g.push_back(d);
+      entries_[g.last].next = id;
+      g.last = id;
+      ++g.count;
       return;
     }
-    launch = it->second.first + 1;
+    launch = g.launch + 1;
+    it.first->second = (int)groups_.size();
   }
-  if ((int)launches_.size() <= launch) launches_.resize(launch + 1);
-  launches_[launch].push_back(StridedSum{d});
-  last_[key] = {launch, (int)launches_[launch].size() - 1};
+  launches_ = std::max(launches_, launch + 1);
+  groups_.push_back(Group{id, id, 1, launch});
 }
 
-void ScatterBatch::run(Context& c) { dev_strided_axpy_launches(c, launches_); }
+void ScatterBatch::run(Context& c) {
+  if (groups_.empty()) return;
+  // the groups by launch, in the order they were opened
+  std::vector<int> ends(launches_, 0);
+  for (const Group& g : groups_) ++ends[g.launch];
+  for (int i = 1; i < launches_; ++i) ends[i] += ends[i - 1];
+  std::vector<int> at(launches_, 0);
+  for (int i = 1; i < launches_; ++i) at[i] = ends[i - 1];
+  std::vector<const Group*> order(groups_.size());
+  for (const Group& g : groups_) order[at[g.launch]++] = &g;
+  std::vector<StridedAxpy> desc;
+  desc.reserve(entries_.size());
+  std::vector<StridedSum> sums;
+  sums.reserve(groups_.size());
+  for (const Group* g : order) {
+    sums.push_back(StridedSum{(int)desc.size(), g->count});
+    for (int e = g->first; e >= 0; e = entries_[e].next) desc.push_back(entries_[e].d);
+  }
+  dev_strided_sums(c, desc, sums, ends);
+}
 
 void dev_scaled_columns(Context& c, const std::vector<ScaledColumns>& jobs) {
   ScaleArgs args;

@@ -1,7 +1,7 @@
 // Small device building blocks shared by the SVD, environment and driver code.
 #pragma once
 
-#include <map>
+#include <unordered_map>
 #include <tuple>
 #include <vector>
 
@@ -38,8 +38,19 @@ class ScatterBatch {
   void run(Context& c);
 
  private:
-  std::map<const void*, std::pair<int, int>> last_;   // key -> launch and group of its last entry
-  std::vector<std::vector<StridedSum>> launches_;
+  // entries in order of add(), each naming the next of its group (-1: the
+  // last); one flat list, since a step adds thousands of them
+  struct Entry {
+    StridedAxpy d;
+    int next;
+  };
+  struct Group {
+    int first, last, count, launch;
+  };
+  std::vector<Entry> entries_;
+  std::vector<Group> groups_;
+  std::unordered_map<const void*, int> last_;   // key -> its last group
+  int launches_ = 0;
 };
 
 // dst[:, j] = f[j] * src[:, j] for the cols columns of rows contiguous
