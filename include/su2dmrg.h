@@ -212,8 +212,9 @@ int su2_heff_set_kernel_path(su2_ctx* ctx, su2_heff* plan, int uniform, int* lay
  * number; *discarded the summed squares of the cut values.  With max_dcut at
  * least the columns of all sectors together nothing can be cut, and U and V
  * hold every direction down to the rounding level: such a call uses the plain
- * Jacobi iteration throughout (two to six times slower), so that those
- * directions stay what they have been. */
+ * Jacobi iteration throughout (two to eight times slower).  Directions at the
+ * rounding level are whatever an iteration leaves, either way; where a cut falls
+ * among them, sectors give them up in proportion, by their norms. */
 int su2_svd_truncate(su2_ctx* ctx, const su2_tensor* psi, double p1, double p2, int max_dcut,
                      su2_tensor** U, su2_tensor** V, double* kept, int cap, int* nkept,
                      double* discarded);

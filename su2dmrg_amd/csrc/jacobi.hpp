@@ -15,24 +15,25 @@
 // Columns are cut into blocks of 16 (or 32), and before each sweep they are put
 // in descending norm order.  Two iterations rotate them:
 //
-// The usual one starts from QR-preconditioned columns (precond.hpp: every
-// block under 256 columns, and from the caller's limit on; what the first
-// pass leaves below 3e-8 of the block a second time).  A sweep begins with the
-// Gram matrix of the columns above the rounding level, which says which pairs
-// of column blocks still need a rotation; only those are visited, in rounds
-// of disjoint pairs, with three launches per round: partial Gram matrices of
-// the pairs over row slices of W, one workgroup per pair that diagonalises
+// The usual one starts from QR-preconditioned columns (precond.hpp; blocks from
+// the caller's limit on, and with a limit up to 256 the smaller ones too).  A
+// sweep begins with the Gram matrix of the columns above the rounding level,
+// which says which pairs of column blocks still need a rotation; only those
+// are visited, in rounds of disjoint pairs, with three launches per round:
+// partial Gram matrices of the pairs over row slices of W, one workgroup per
+// pair that diagonalises
 // its (up to 64 x 64) Gram matrix in LDS by parallel cyclic Jacobi, p columns
 // against q columns (all of them in a block's first visit), and the pairs'
 // columns of W times the result (V's a round later, beside the next
-// diagonalisations).  A block is done when no pair needs a rotation.
+// diagonalisations).  A block is done when no pair needs a rotation, or when
+// every scheduled pair passed the launch's own test, on sums in another order.
 //
 // The plain one visits every pair once per sweep with two launches per round
 // (Gram matrices, then every row slice diagonalises the whole pair for itself
 // and rotates its rows of W and V), preconditioned from the caller's limit on
 // only.  It is kept for uncut SVD calls (svd.hpp says why).  Measured against
-// it: svd call of a d = 500 step 20.7 -> 9.6 ms, d = 2000 83 -> 47 ms; 192 x
-// 192 block 14.1 -> 5.2 ms.
+// it: svd call of a d = 500 step 20.6 -> 7.8 ms, d = 2000 84 -> 45 ms; a 192 x
+// 192 block 13.3 -> 3.7 ms, 1390 x 1383 of rank 1106 66 -> 35 ms.
 //
 // Sweeps stop when every pair is orthogonal to
 // |g_ij| <= max(tol * sqrt(g_ii g_jj), 1e-14 ||A||_F (sqrt g_ii + sqrt g_jj))
@@ -64,7 +65,8 @@ struct JacobiBlock {
                            // each other's bits
 };
 
-// Decomposes every block and returns the number of sweeps it took.  W and V columns are sorted ascending by singular value; each
+// Decomposes every block and returns the number of sweeps it took.  W and V
+// columns are sorted ascending by singular value; each
 // column of V has its first entry with |v| >= max|v|/2 made positive (the
 // LAPACK routine the reference calls leaves signs open), W's columns follow.
 // block_cols: 16 (pairs of 32 columns, one wave per pair) or 32 (pairs of 64

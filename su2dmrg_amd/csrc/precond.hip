@@ -319,8 +319,8 @@ __global__ __launch_bounds__(PT) void wy_panel_kernel(const PDesc* __restrict__ 
   }
 }
 
-// Householder QR of one 16-column panel of X for the plain iteration, which
-// keeps every direction down to rounding and its bits (rows c0..K-1; row c0 + r on
+// Householder QR of one 16-column panel of X for the plain iteration, reflector
+// by reflector (rows c0..K-1; row c0 + r on
 // thread r % 1024, in registers).
 // Column j becomes its Householder vector below the diagonal (the unit
 // diagonal implicit); the panel's T factor of the compact WY form H_0 ...

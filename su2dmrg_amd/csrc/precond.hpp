@@ -42,7 +42,7 @@ constexpr int kPrecondMaxK = 2048;
 
 // Preconditions every block (each must have 1 <= K <= kPrecondMaxK and
 // L >= K): Wout = W Q2, Vout = V Q2.  Blocks never affect each other's bits.
-// plain: reflectors column by column (the plain iteration's bits).
+// plain: reflectors one by one (hh_panel_kernel), for the plain iteration.
 void precondition_jacobi(Context& c, std::vector<PrecondBlock>& blocks, bool plain);
 
 }  // namespace su2

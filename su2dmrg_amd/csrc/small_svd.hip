@@ -1,12 +1,13 @@
 // One-sided Jacobi SVD in LDS, see small_svd.hpp.
 //
 // The columns of W (the block or its transpose, L x k with L >= k) and of V (k x k, from the
-// identity) are stacked in LDS.  First W is made lower trapezoidal by Householder reflectors from
-// the right, each for the row with the largest remaining norm (W Q is then the transposed R factor
-// of a QR with column pivoting of W^T, on which Jacobi converges fast after Drmac and Veselic; V
-// becomes Q).  Then pairs of columns are rotated until orthogonal (Hestenes): a sweep has k - 1
-// round-robin rounds of k / 2 disjoint pairs, a group of lanes owns a pair for one round, and one
-// barrier separates two rounds.  Nothing else does: no launch, no Gram matrix, no host wait.
+// identity) are stacked in LDS, longest columns first.  Then W is made lower trapezoidal by
+// Householder reflectors from the right, each for the row with the largest remaining norm (W Q is
+// then the transposed R factor of a QR with column pivoting of W^T, on which Jacobi converges fast
+// after Drmac and Veselic; V becomes Q).  Last, pairs of columns are rotated until orthogonal
+// (Hestenes): a sweep has k - 1 round-robin rounds of k / 2 disjoint pairs, a group of lanes owns a
+// pair for one round, and one barrier separates two rounds.  Nothing else does: no launch, no Gram
+// matrix, no host wait.
 // Columns are never reordered between sweeps: after the reflectors they come in nearly descending
 // order, and a model of the iteration took 7 sweeps without reordering at k = 44, 8 with it, 24
 // without the reflectors (7, 9 and more than 20 at k = 120).
@@ -20,7 +21,7 @@
 // k = 42 (clock stamps): 4150 cycles per reflector, 7 sweeps of 41 rounds at 1620 cycles, of which
 // 416 wait for the columns (LDS bandwidth: both columns of every pair pass through it each round),
 // 75 form the dot product, 290 the rotation, the rest updates, drains and waits for the slowest
-// wave.  The SVD call of a d = 64 step: 2.95 ms by pairs of 32-column blocks, 0.47 ms here.
+// wave.  The SVD call of a d = 64 step: 2.95 ms by pairs of 32-column blocks, 0.36 ms here.
 #include "small_svd.hpp"
 
 #include <algorithm>

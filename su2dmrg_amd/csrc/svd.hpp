@@ -2,14 +2,13 @@
 // (tensor_su2::svd, tensor_su2.cpp:1619-1758, with tensor::svd per sector,
 // tensor.cpp:1472-1700).
 //
-// Per sector j with block A (m x n): the Gram matrix A^T A (m >= n) or A A^T
-// is formed with the grouped FP64 MFMA GEMM and diagonalised on the device;
-// eigenpairs with w/w_max < 0.1 are re-diagonalised in their projected Gram
-// until one remains (tensor.cpp:1498-1529); the other factor is A V (or
-// A^T U); singular values are sqrt(w) for w/w_max > 1e-100; kept columns are
-// scaled by s^(p1-1)/s^p2 (or s^p1/s^(p2-1)).  The largest max_dcut values
-// over all sectors survive, ordered by the reference's shell sort so ties at
-// the cut fall the same way (sort2.f:76-111).
+// Per sector j with block A (m x n): a one-sided Jacobi SVD (jacobi.hpp) of its
+// short side's columns, where the reference diagonalises the Gram matrix again
+// and again (tensor.cpp:1498-1529); singular values count for w/w_max > 1e-100,
+// w = s^2; kept columns are scaled by s^(p1-1)/s^p2 (or s^p1/s^(p2-1)).  The
+// largest max_dcut values over all sectors survive, ordered by the reference's
+// shell sort so ties at the cut fall the same way (sort2.f:76-111); values at
+// the rounding level of their sector are ordered by its norm alone.
 #pragma once
 
 #include <memory>
@@ -36,13 +35,16 @@ struct SvdResult {
 };
 
 // keep_all_plain: where nothing can be cut (max_dcut >= the columns of all
-// sectors together), use the plain Jacobi iteration (JacobiBlock, plain).  Such
-// a result holds every direction down to the rounding level, where it is
-// whatever the iteration leaves; this keeps it what it has always been for a
-// caller that stores or compares the factors.  The plain iteration is two to
-// six times slower (d = 2000 step 83 ms against 47, d = 64 step 2.95 against
-// 0.47), so the DMRG solves, whose energies do not depend on those
-// directions, never ask for it.
+// sectors together), use the plain Jacobi iteration (jacobi.hpp).  Such a
+// result holds every direction down to the rounding level, where it is
+// whatever the iteration leaves; the plain one is kept for callers that store
+// or compare the factors, and gives them to rounding as it always has where
+// the singular values determine them.  It is two to eight times slower (d =
+// 2000 step 84 ms against 45, d = 64 step 2.95 against 0.36), and the DMRG
+// solves never ask for it.  They keep null directions too, whenever they keep
+// more multiplets than the state has, and grow into them: which ones those are
+// changes the way of a run (its first sweep's energy by up to a percent on wide
+// cylinders, with any kernel or tuning), not what it converges to.
 SvdResult truncated_svd(Context& c, const Tensor& psi, double p1, double p2, int max_dcut,
                         bool keep_all_plain = false);
 
