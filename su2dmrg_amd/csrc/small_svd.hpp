@@ -13,7 +13,7 @@ struct JacobiBlock;
 // Whether an m x n block is decomposed by small_svd_batched: its columns and
 // its accumulated rotations fit the LDS of one CU (up to 96 x 96, or 128 rows
 // and about 75 columns), the most the kernel takes.  There it is the faster
-// one throughout (whole SVD call, 32 x 32: 0.26 ms against 2.06 ms by pairs
+// one throughout (whole SVD call, 32 x 32: 0.24 ms against 2.06 ms by pairs
 // of column blocks; 64 x 64: 0.61 against 3.8; 96 x 96: 1.73 against 7.9).
 // Depends on the block's shape alone.
 bool small_svd_fits(int m, int n);
