@@ -754,6 +754,15 @@ size_t elem_size(Prec p) { return p == Prec::F64 ? sizeof(double) : sizeof(float
 
 int gemm_num_variants(Prec p) { return num_variants(p); }
 
+// unsigned 32-bit byte offsets, plus one tile of margin past the M / N edge
+bool gemm_slice_fits(Prec p, int M, int N, int K, long long lda, int transA, long long ldb,
+                     int transB) {
+  const long long lim = (1LL << 32) / (long long)elem_size(p) - 1;
+  const long long a_span = transA ? (long long)(M + 256) * lda + K : (long long)(K + 256) * lda + M;
+  const long long b_span = transB ? (long long)(K + 256) * ldb + N : (long long)(N + 256) * ldb + K;
+  return a_span < lim && b_span < lim;
+}
+
 GroupedGemm::~GroupedGemm() { release(); }
 
 void GroupedGemm::release() {
@@ -793,12 +802,7 @@ void GroupedGemm::add_slice(int problem, const void* A, long long lda, int trans
   SU2_CHECK(K > 0, kErrArgument, "gemm: empty slice");
   SU2_CHECK(lda >= (transA ? K : std::max(p.M, 1)) && ldb >= (transB ? std::max(p.N, 1) : K),
             kErrArgument, "gemm: leading dimension too small");
-  // the kernel addresses a slice with unsigned 32-bit byte offsets (plus one
-  // tile of margin past the M / N edge)
-  const long long lim = (1LL << 32) / (long long)elem_size(prec_) - 1;
-  const long long a_span = transA ? (long long)(p.M + 256) * lda + K : (long long)(K + 256) * lda + p.M;
-  const long long b_span = transB ? (long long)(K + 256) * ldb + p.N : (long long)(p.N + 256) * ldb + K;
-  SU2_CHECK(a_span < lim && b_span < lim, kErrCapacity,
+  SU2_CHECK(gemm_slice_fits(prec_, p.M, p.N, K, lda, transA, ldb, transB), kErrCapacity,
             "gemm: slice matrix over 4 GB (M=%d N=%d K=%d)", p.M, p.N, K);
   GemmSlice sl{};
   sl.A = A;

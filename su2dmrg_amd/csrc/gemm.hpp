@@ -63,6 +63,10 @@ struct ReduceProblem {
 
 // Number of compiled tile variants (BM x BN x BK x waves) of a precision.
 int gemm_num_variants(Prec p = Prec::F64);
+// Whether a slice's operands are within the kernel's 32-bit byte offsets (4 GB
+// each, with one tile of margin); add_slice takes no others.
+bool gemm_slice_fits(Prec p, int M, int N, int K, long long lda, int transA, long long ldb,
+                     int transB);
 
 // Host-side plan: build problems, then finalize once; launch many times.
 class GroupedGemm {

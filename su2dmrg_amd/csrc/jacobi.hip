@@ -1771,14 +1771,26 @@ int jacobi_svd_batched(Context& c, std::vector<JacobiBlock>& blocks, double tol,
                        int precondition_min_k, bool plain) {
   // a block's own shape decides, so its bits do not depend on the rest of
   // the batch
-  std::vector<JacobiBlock*> small, large;
-  for (JacobiBlock& b : blocks) (!plain && small_svd_fits(b.m, b.n) ? small : large).push_back(&b);
-  double w1 = 0.0, w2 = 0.0;
+  std::vector<JacobiBlock*> small, large, by_slices;
+  for (JacobiBlock& b : blocks) {
+    const int L = std::max(b.m, b.n), k = std::min(b.m, b.n);
+    if (plain) by_slices.push_back(&b);
+    else if (small_svd_fits(b.m, b.n)) small.push_back(&b);
+    // the usual iteration takes the whole Gram matrix, and W Q2, from grouped
+    // GEMMs, the plain one only row slices of W (2 000 000 x 20 does not fit,
+    // nor about 23000 x 23000)
+    else if (gemm_slice_fits(Prec::F64, k, k, L, L, 1, L, 0) &&
+             gemm_slice_fits(Prec::F64, L, k, k, L, 0, k, 0)) large.push_back(&b);
+    else by_slices.push_back(&b);
+  }
+  double w1 = 0.0, w2 = 0.0, w3 = 0.0;
   const int n1 = small_svd_batched(c, small, tol, kTolAbs, kNoiseRel, max_sweeps, &w1);
   const int n2 = jacobi_svd_large(c, large, tol, max_sweeps, block_cols, inner_sweeps, &w2,
-                                  precondition_min_k, plain);
-  if (worst_out) *worst_out = std::max(w1, w2);
-  return std::max(n1, n2);
+                                  precondition_min_k, false);
+  const int n3 = jacobi_svd_large(c, by_slices, tol, max_sweeps, block_cols, inner_sweeps, &w3,
+                                  precondition_min_k, true);
+  if (worst_out) *worst_out = std::max({w1, w2, w3});
+  return std::max({n1, n2, n3});
 }
 
 }  // namespace su2

@@ -31,7 +31,8 @@
 // The plain one visits every pair once per sweep with two launches per round
 // (Gram matrices, then every row slice diagonalises the whole pair for itself
 // and rotates its rows of W and V), preconditioned from the caller's limit on
-// only.  It is kept for uncut SVD calls (svd.hpp says why).  Measured against
+// only.  It is kept for uncut SVD calls (svd.hpp says why) and for blocks past
+// the grouped GEMM's 4 GB of addresses.  Measured against
 // it: svd call of a d = 500 step 20.6 -> 7.8 ms, d = 2000 84 -> 45 ms; a 192 x
 // 192 block 13.3 -> 3.7 ms, 1390 x 1383 of rank 1106 66 -> 35 ms.
 //
