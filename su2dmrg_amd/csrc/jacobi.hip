@@ -917,7 +917,7 @@ __device__ __forceinline__ void apply_rows(double* __restrict__ M, int rows, con
 
 // The first nj workgroups diagonalise this round's pairs, the others apply
 // the previous round's rotations to V's row tiles (nv of them per pair).
-// moved: one flag per block of the batch (pinned), set where a pair rotated.
+// moved: one flag per block of the batch, set where a pair rotated.
 template <int CB>
 __global__ __launch_bounds__(SolveThreads<CB>::value) void solve_kernel(
     const BlockDesc* __restrict__ blocks, const PairJob* __restrict__ jobs, int nj, int pmax,
@@ -1054,11 +1054,13 @@ __device__ __forceinline__ int col_block(const long long* __restrict__ noff, int
 }
 
 // squared column norms of every block's current W into out[0, ncol) and of
-// its V into out[ncol, 2 ncol) (one workgroup per column)
+// its V into out[ncol, 2 ncol) (one workgroup per column); every block's flag
+// into out[2 ncol, 2 ncol + nb) and back to zero
 __global__ __launch_bounds__(256) void colnorm_batched_kernel(const BlockDesc* __restrict__ desc,
                                                               const long long* __restrict__ noff,
                                                               int nb, long long ncol,
-                                                              double* __restrict__ out) {
+                                                              double* __restrict__ out,
+                                                              int* __restrict__ moved) {
   __shared__ double s[2][256];
   const long long gc = blockIdx.x;
   const int b = col_block(noff, nb, gc);
@@ -1081,6 +1083,10 @@ __global__ __launch_bounds__(256) void colnorm_batched_kernel(const BlockDesc* _
   if (threadIdx.x == 0) {
     out[gc] = s[0][0];
     out[ncol + gc] = s[1][0];
+    if (gc == noff[b]) {
+      out[2 * ncol + b] = moved[b] != 0;
+      moved[b] = 0;
+    }
   }
 }
 
@@ -1260,14 +1266,18 @@ static int jacobi_svd_large(Context& c, const std::vector<JacobiBlock*>& blocks,
     SU2_HIP(hipMemcpyAsync(dtab.p, tab.data(), tab.size(), hipMemcpyHostToDevice, st));
   };
   // squared column norms of the current W and V of every block, written to
-  // pinned memory by the kernel
+  // pinned memory by the kernel, and whether any of a block's pairs rotated
+  // since the last call (nothing before the first; every block has a column)
+  DevMem dmoved(c, sizeof(int) * nb);
+  std::vector<char> rotated(nb, 0);
   auto norms = [&]() {
-    double* h = c.host_scratch(2 * ncol);
+    double* h = c.host_scratch(2 * ncol + nb);
     hipLaunchKernelGGL(colnorm_batched_kernel, dim3((unsigned)ncol), dim3(256), 0, st, ddesc,
-                       (const long long*)dnoff.p, nb, (long long)ncol, h);
+                       (const long long*)dnoff.p, nb, (long long)ncol, h, (int*)dmoved.p);
     SU2_HIP(hipGetLastError());
     SU2_HIP(hipStreamSynchronize(st));
     std::memcpy(hn.data(), h, sizeof(double) * 2 * ncol);
+    for (int b = 0; b < nb; ++b) rotated[b] = h[2 * ncol + b] != 0.0;
   };
   // src -> dst column moves of W and V: the first n jobs of the table
   // (prepare_permute before the upload, permute after it)
@@ -1657,7 +1667,7 @@ static int jacobi_svd_large(Context& c, const std::vector<JacobiBlock*>& blocks,
     const int wt = (lmax + rows_per_tile - 1) / rows_per_tile;
     const int vt = (kmax + rows_per_tile - 1) / rows_per_tile;
     // each round's three launches, and a last one for V's rotations of the last round
-    auto run_rounds = [&](auto cb, int* moved) {
+    auto run_rounds = [&](auto cb) {
       constexpr int B = decltype(cb)::value;
       constexpr int NT = SolveThreads<B>::value;
       const BlockDesc* dd = ddesc;
@@ -1682,7 +1692,7 @@ static int jacobi_svd_large(Context& c, const std::vector<JacobiBlock*>& blocks,
         if (nj + nprev > 0)
           hipLaunchKernelGGL(solve_kernel<B>, dim3(nj + nprev * vt), dim3(NT), 0, st, dd, jr, nj,
                              pm, (const double*)dgpart.p, tol, kTolAbs, inner_sweeps, rot, act,
-                             moved, prev, vt, prot, pact);
+                             (int*)dmoved.p, prev, vt, prot, pact);
         if (nj > 0)
           hipLaunchKernelGGL(apply_kernel<B>, dim3(nj * wt), dim3(NT), 0, st, dd, jr, wt,
                              (const double*)rot, (const int*)act);
@@ -1704,13 +1714,11 @@ static int jacobi_svd_large(Context& c, const std::vector<JacobiBlock*>& blocks,
       // summed in another order.  A pair at the threshold can pass there, so a
       // block whose pairs all passed is done: nothing would change in the next
       // sweep, nor its flags.
-      int* moved = (int*)(c.host_scratch(2 * ncol + nb) + 2 * ncol);
-      std::fill(moved, moved + nb, 0);
-      if (CB == 16) run_rounds(std::integral_constant<int, 16>{}, moved);
-      else run_rounds(std::integral_constant<int, 32>{}, moved);
+      if (CB == 16) run_rounds(std::integral_constant<int, 16>{});
+      else run_rounds(std::integral_constant<int, 32>{});
       norms();
       for (int b = 0; b < nb; ++b)
-        if (!moved[b]) active[b] = 0;
+        if (!rotated[b]) active[b] = 0;
     }
   }
   // Out of sweeps: the columns are accepted when orthogonal to 1e-6 of their
